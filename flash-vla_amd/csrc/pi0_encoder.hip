@@ -3,13 +3,10 @@
 // At these shapes the GEMMs are MFMA-bound (2 * 768 * 2048 * 32768 flops for the
 // gated FFN alone), so the design is the classic LDS-tiled one:
 //   * tile_gemm_kernel<BM, BN, EPI, DUAL>: 4 waves in a 2 x 2 grid, BM x BN
-//     output block, K consumed 64 at a time through two LDS stages. Both
-//     operands are kept in LDS in MFMA fragment order (one 1 KB slot per
-//     16 x 32 fragment: lane-contiguous 16-byte reads, free of bank conflicts):
-//     A (row-major activations) is loaded one fragment per instruction straight
-//     from global memory, B is the packed weight stream, already in that order.
-//     While a stage is multiplied, the next stage's fragments are in flight in
-//     registers; one barrier per 64-deep step.
+//     output block, K consumed 64 at a time through a ring of steps. A (row-major
+//     activations) goes to LDS in whole 128-byte step rows, 16-byte chunks
+//     XOR-swizzled by row; B is the packed weight stream, already in MFMA
+//     fragment order. One barrier per 64-deep step.
 //   * tiles are assigned so that the workgroups dispatched to one XCD (the
 //     hardware deals workgroups round-robin over the 8 XCDs) cover consecutive
 //     tiles -- all row blocks of a weight column block -- so each weight block
@@ -71,9 +68,15 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
 // Workgroup = 4 waves side by side along N; each wave owns all BM rows of the
 // block and WN of its B columns. Both operands run D 64-deep steps ahead:
 //   * A (activations, shared by the 4 waves) goes global -> LDS directly
-//     (buffer_load ... lds, 16 bytes per lane, one MFMA fragment per
-//     instruction) into a D-slot ring; the buffer resource ends at row M so the
-//     rows of a ragged last block load as zeros;
+//     (buffer_load ... lds, 16 bytes per lane) into a D-slot ring; the buffer
+//     resource ends at row M so the rows of a ragged last block load as zeros.
+//     An instruction reads 8 rows x 128 bytes, whole cache lines: reading one
+//     32 x 16 fragment instead (32 lines, 32 bytes of each, every line touched by
+//     four instructions) held the load path back. Encoder down at M = 768 71.6 ->
+//     58.8 us, o-proj 18.4 -> 15.4, vision QKV 14.2 -> 11.8, FFN-up 20.8 -> 18.0;
+//     vision at 3072 rows QKV 47.6 -> 36.2, FFN-down 54.8 -> 43.9. The swizzle
+//     (chunk c of row r sits at c ^ (r % 8)) keeps the fragment reads of 8
+//     neighbouring rows on distinct banks;
 //   * B (the packed weight stream, private to the wave) goes global -> VGPRs
 //     into a D-slot register ring, so no weight byte passes through LDS.
 // The step count is a multiple of D (the host checks), so the ring unrolls with
@@ -123,12 +126,13 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(TileArgs a) {
   const int arows = max(min(BM, a.M - m0), 0);
   const __amdgpu_buffer_rsrc_t ar =
       rows_rsrc_sgpr(a.a + (size_t)m0 * a.lda, arows * a.lda * (int)sizeof(__bf16));
-  int aoff[LA];
-#pragma unroll
-  for (int i = 0; i < LA; ++i) {
-    const int q = i * 4 + wave, rt = q >> 2, kq = q & 3;   // A fragment q = rt * 4 + kq
-    aoff[i] = ((rt * 32 + (lane & 31)) * a.lda + kq * 16 + (lane >> 5) * 8) * (int)sizeof(__bf16);
-  }
+  // copy i of wave w covers block rows (4 i + w) * 8 .. + 7 whole 128-byte step rows (full
+  // cache lines); LDS word (row, c) receives the row's 16-byte chunk c ^ (row % 8)
+  const int aoff = ((wave * 8 + (lane >> 3)) * a.lda + ((lane & 7) ^ (lane >> 3)) * 8) *
+                   (int)sizeof(__bf16);
+  const int arow_step = 32 * a.lda * (int)sizeof(__bf16);
+  // ... so this lane's piece of A fragment (row tile i, slice kq) is word i * 256 + (afrag ^ 2 kq)
+  const int afrag = (lane & 31) * 8 + ((lane >> 5) ^ (lane & 7));
   // this wave's 32-column B tiles: for the gated FFN, FN / 2 gate tiles then FN / 2 up tiles
   const __bf16* bptr[FN];
 #pragma unroll
@@ -156,7 +160,7 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(TileArgs a) {
     const int abase = st * 64 * (int)sizeof(__bf16);
 #pragma unroll
     for (int i = 0; i < LA; ++i)
-      buf_load16_lds(ar, &lds[(slot * TA + i * 4 + wave) * 64], aoff[i] + abase);
+      buf_load16_lds_s(ar, &lds[(slot * TA + i * 4 + wave) * 64], aoff, abase + i * arow_step);
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
@@ -210,13 +214,13 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(TileArgs a) {
       const bf16x8* st = lds + u * TA * 64;
       bf16x8 ap[PF];
 #pragma unroll
-      for (int p = 0; p < PF - 1; ++p) ap[p] = st[((p % FM) * 4 + p / FM) * 64 + lane];
+      for (int p = 0; p < PF - 1; ++p) ap[p] = st[(p % FM) * 256 + (afrag ^ (p / FM * 2))];
 #pragma unroll
       for (int f = 0; f < 4 * FM; ++f) {
         const int kq = f / FM, i = f % FM;
         if (f + PF - 1 < 4 * FM) {
           const int fn = f + PF - 1;
-          ap[(f + PF - 1) % PF] = st[((fn % FM) * 4 + fn / FM) * 64 + lane];
+          ap[(f + PF - 1) % PF] = st[(fn % FM) * 256 + (afrag ^ (fn / FM * 2))];
         }
         __builtin_amdgcn_sched_barrier(0);   // keep the prefetch ahead of these MFMAs
 #pragma unroll
@@ -367,7 +371,7 @@ __global__ __launch_bounds__(64 * NW, 1) void tile2_gated_kernel(TileArgs a) {
   constexpr int OUTC = 128, OP = OUTC + 8; // output columns, bf16 pitch of the parked tile
   constexpr int PARK = (BM * OP * 2 + 15) / 16;
   static_assert(BM % (32 * WMR) == 0 && TA % NW == 0 && TB % NW == 0 && D >= 2, "tile shape");
-  static_assert(NW % KS == 0 && 4 % CPW == 0, "copy assignment");
+  static_assert(KS == 4 && NW % KS == 0 && 4 % CPW == 0, "copy assignment");
   __shared__ bf16x8 lds[D * SLOT > PARK ? D * SLOT : PARK];
 
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -387,14 +391,16 @@ __global__ __launch_bounds__(64 * NW, 1) void tile2_gated_kernel(TileArgs a) {
   const int wbytes = 4 * KT * 512 * (int)sizeof(__bf16);
   const __amdgpu_buffer_rsrc_t gr = rows_rsrc_sgpr(a.w0 + (size_t)ntile * 4 * KT * 512, wbytes);
   const __amdgpu_buffer_rsrc_t ur = rows_rsrc_sgpr(a.w1 + (size_t)ntile * 4 * KT * 512, wbytes);
-  // copy i of wave w is fragment q = i * NW + w of each operand (q = tile * KS + slice,
-  // slice w % KS, tile i * CPW + w / KS); the i-dependent parts of the offsets are
+  // copy q = i * NW + w of wave w is, of A, block rows 8 q .. 8 q + 7 (whole 128-byte step
+  // rows, chunks swizzled as in the strip kernel) and, of B, fragment q = tile * KS + slice
+  // (slice w % KS, tile i * CPW + w / KS); the i-dependent parts of the offsets are
   // wave-uniform (scalar), so each operand needs one lane offset
-  const int avoff = (((wave / KS) * 32 + (lane & 31)) * a.lda + (wave % KS) * 16 + (lane >> 5) * 8) *
+  const int avoff = ((wave * 8 + (lane >> 3)) * a.lda + ((lane & 7) ^ (lane >> 3)) * 8) *
                     (int)sizeof(__bf16);
+  const int afrag = (lane & 31) * 8 + ((lane >> 5) ^ (lane & 7));
   const int btile = KT * 512 * (int)sizeof(__bf16);
   const int bvoff = ((wave % KS) * 512 + lane * 8) * (int)sizeof(__bf16) + (wave / KS) * btile;
-  const int arow_step = CPW * 32 * a.lda * (int)sizeof(__bf16);
+  const int arow_step = NW * 8 * a.lda * (int)sizeof(__bf16);
 
   auto issue = [&](int s, int slot) {
     const int abase = s * KS * 16 * (int)sizeof(__bf16);
@@ -442,7 +448,7 @@ __global__ __launch_bounds__(64 * NW, 1) void tile2_gated_kernel(TileArgs a) {
         }
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
-          const bf16x8 af = st[((wm * FM + i) * KS + kq) * 64 + lane];
+          const bf16x8 af = st[(wm * FM + i) * 256 + (afrag ^ (kq * 2))];
 #pragma unroll
           for (int j = 0; j < FN; ++j) acc[i][j] = mfma32(af, bf[j], acc[i][j]);
         }
