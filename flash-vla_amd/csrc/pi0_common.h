@@ -61,6 +61,19 @@ __device__ __forceinline__ float gelu_tanh(float v) {
   const float c0 = 1.5957691216057308f, c1 = 0.044715f;
   return v / (1.0f + __expf(-(c0 * v * (1.0f + c1 * v * v))));
 }
+// The same in fewer instructions, for the encoder and vision tiles, whose epilogues are
+// bound by them: v / (1 + 2^a) with a = v (k0 + k1 v^2), k0 = -c0 log2 e, k1 = c1 k0, the
+// quotient as v * rcp(d) with one residual correction and the division's own handling of
+// zeros, infinities and NaN. 16 issue slots against 25; the old form was 12% of a gated
+// FFN block's clocks. Relative error in the 2-norm against 64 bits: 4.06e-8 over
+// [-0.5, 0.5], 2.23e-8 over [-8, 8] (gelu_tanh: 4.21e-8 and 2.24e-8).
+__device__ __forceinline__ float gelu_tanh_rcp(float v) {
+  const float k0 = -2.3022082f, k1 = -0.10294324f;
+  const float d = 1.0f + fast_exp2(v * fmaf(v * v, k1, k0));
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float y = v * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, y, v), r, y), d, v);
+}
 __device__ __forceinline__ float silu(float v) { return v / (1.0f + __expf(-v)); }
 
 // ---- bounds-checked row loads ---------------------------------------------------

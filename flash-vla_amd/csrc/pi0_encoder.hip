@@ -271,7 +271,8 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(TileArgs a) {
 #pragma unroll
           for (int j = 0; j < FN / 2; ++j)
             cs[row * CP + (wave * (FN / 2) + j) * 32 + r] =
-                gelu_tanh(fr * acc[i][j][e]) * (fr * acc[i][FN / 2 + j][e]);
+                RMS ? gelu_tanh(fr * acc[i][j][e]) * (fr * acc[i][FN / 2 + j][e])
+                    : gelu_tanh_rcp(acc[i][j][e]) * acc[i][FN / 2 + j][e];
         } else {
 #pragma unroll
           for (int j = 0; j < FN; ++j) cs[row * CP + (wave * FN + j) * 32 + r] = acc[i][j][e];
@@ -337,7 +338,7 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(TileArgs a) {
       }
       if constexpr (EPI == TE_BIAS_GELU) {
 #pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = gelu_tanh(v[q]);
+        for (int q = 0; q < 8; ++q) v[q] = gelu_tanh_rcp(v[q]);
       }
     }
     bf16x8 o;
@@ -472,7 +473,7 @@ __global__ __launch_bounds__(64 * NW, 1) void tile2_gated_kernel(TileArgs a) {
         const int row = (wm * FM + i) * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          cs[row * OP + wn * 64 + j * 32 + r] = f2bf(gelu_tanh(acc[i][j][e]) * acc[i][2 + j][e]);
+          cs[row * OP + wn * 64 + j * 32 + r] = f2bf(gelu_tanh_rcp(acc[i][j][e]) * acc[i][2 + j][e]);
       }
   }
   __syncthreads();
