@@ -228,7 +228,7 @@ def main_encoder(args, torch):
                 ck["encoder_ffn_up_w"][i % ENC_LAYERS], b["encoder_hidden"], b["encoder_x_norm"]),
                 n_inner=ENC_LAYERS, reps=10, torch=torch)
         achieved = gate_flops / (us * 1e-6) / 1e12
-        roof = {"kernel": "tile2_gated_kernel + rms_norm_kernel (encoder_norm_gated_ffn)",
+        roof = {"kernel": "block_gemm_kernel + rms_norm_kernel (encoder_norm_gated_ffn)",
                 "bound": "mfma", "achieved": round(achieved, 1), "peak": MFMA_BF16_PEAK_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(achieved / MFMA_BF16_PEAK_TFLOPS, 4),
                 "traffic": int(ENC_GATE_TRAFFIC_BYTES), "avg_launch_us": round(us, 3), "flops_per_launch": gate_flops}
@@ -302,7 +302,7 @@ def main_full(args, torch):
                 n_inner=ENC_LAYERS, reps=10, torch=torch)
         gate_flops = 2 * M_enc * ENC_W * 2 * ENC_FFN
         achieved = gate_flops / (us * 1e-6) / 1e12
-        roof = {"kernel": "tile2_gated_kernel + rms_norm_kernel (encoder_norm_gated_ffn)",
+        roof = {"kernel": "block_gemm_kernel + rms_norm_kernel (encoder_norm_gated_ffn)",
                 "bound": "mfma", "achieved": round(achieved, 1), "peak": MFMA_BF16_PEAK_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(achieved / MFMA_BF16_PEAK_TFLOPS, 4),
                 "traffic": int(ENC_GATE_TRAFFIC_BYTES) if not config5 else None,

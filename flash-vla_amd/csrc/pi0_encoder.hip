@@ -27,6 +27,10 @@
 #include "pi0_common.h"
 #include "pi0_hip.h"
 
+#include <algorithm>
+#include <cmath>
+#include <initializer_list>
+
 namespace pi0 {
 
 enum TileEpi {
@@ -56,6 +60,60 @@ struct TileArgs {
 
 __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Epilogue of 8 consecutive columns col .. col + 7 of output row grow: v holds the fp32
+// products, b8 / r8 the bias and residual pieces (where the form has them).
+template <int EPI>
+__device__ __forceinline__ void tile_store(const TileArgs& a, int grow, int col, float* v, bf16x8 b8,
+                                           bf16x8 r8) {
+  __bf16* dst;
+  if constexpr (EPI == TE_QKV_ROPE) {
+    const int hd = a.head_dim, qdim = a.heads * hd;
+    const int bq = grow / a.rows_per_batch, tq = grow - bq * a.rows_per_batch;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = round_bf(v[q]);
+    if (col < qdim + hd) {          // rotate the rounded pairs (2p, 2p + 1)
+      const bf16x8 rp = load8(a.rope + (size_t)tq * hd + (col % hd));
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const float cs_ = bf2f(rp[2 * p]), sn = bf2f(rp[2 * p + 1]);
+        const float x0 = v[2 * p], x1 = v[2 * p + 1];
+        v[2 * p] = x0 * cs_ - x1 * sn;
+        v[2 * p + 1] = x1 * cs_ + x0 * sn;
+      }
+    }
+    const size_t kv = (size_t)bq * a.kv_bstride + (size_t)tq * a.ldkv;
+    if (col < qdim) dst = a.out + (size_t)grow * qdim + col;
+    else if (col < qdim + hd) dst = a.out_k + kv + (col - qdim);
+    else dst = a.out_v + kv + (col - qdim - hd);
+  } else {
+    dst = a.out + (size_t)grow * a.ldo + col;
+    if constexpr (EPI == TE_BIAS) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] += bf2f(b8[q]);
+    }
+    if constexpr (EPI == TE_RES) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] += bf2f(r8[q]);
+    }
+    if constexpr (EPI == TE_BIAS_RES || EPI == TE_BIAS_GELU) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] += bf2f(b8[q]);
+    }
+    if constexpr (EPI == TE_BIAS_RES) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] += bf2f(r8[q]);
+    }
+    if constexpr (EPI == TE_BIAS_GELU) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = gelu_tanh_rcp(v[q]);
+    }
+  }
+  bf16x8 o;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) o[q] = f2bf(v[q]);
+  *reinterpret_cast<bf16x8*>(dst) = o;
 }
 
 // v_mfma_f32_32x32x16_bf16 is used because one wave per SIMD sustains ~90% of the
@@ -298,124 +356,89 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(TileArgs a) {
       *reinterpret_cast<f32x4*>(dst + 4) = hi;
       continue;
     }
-    __bf16* dst;
-    if constexpr (EPI == TE_QKV_ROPE) {
-      const int hd = a.head_dim, qdim = a.heads * hd;
-      const int bq = grow / a.rows_per_batch, tq = grow - bq * a.rows_per_batch;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = round_bf(v[q]);
-      if (col < qdim + hd) {          // rotate the rounded pairs (2p, 2p + 1)
-        const bf16x8 rp = load8(a.rope + (size_t)tq * hd + (col % hd));
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-          const float cs_ = bf2f(rp[2 * p]), sn = bf2f(rp[2 * p + 1]);
-          const float x0 = v[2 * p], x1 = v[2 * p + 1];
-          v[2 * p] = x0 * cs_ - x1 * sn;
-          v[2 * p + 1] = x1 * cs_ + x0 * sn;
-        }
-      }
-      const size_t kv = (size_t)bq * a.kv_bstride + (size_t)tq * a.ldkv;
-      if (col < qdim) dst = a.out + (size_t)grow * qdim + col;
-      else if (col < qdim + hd) dst = a.out_k + kv + (col - qdim);
-      else dst = a.out_v + kv + (col - qdim - hd);
-    } else {
-      dst = a.out + (size_t)grow * a.ldo + col;
-      if constexpr (EPI == TE_BIAS) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] += bf2f(epb[k][q]);
-      }
-      if constexpr (EPI == TE_RES) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] += bf2f(epr[k][q]);
-      }
-      if constexpr (EPI == TE_BIAS_RES || EPI == TE_BIAS_GELU) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] += bf2f(epb[k][q]);
-      }
-      if constexpr (EPI == TE_BIAS_RES) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] += bf2f(epr[k][q]);
-      }
-      if constexpr (EPI == TE_BIAS_GELU) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = gelu_tanh_rcp(v[q]);
-      }
-    }
-    bf16x8 o;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) o[q] = f2bf(v[q]);
-    *reinterpret_cast<bf16x8*>(dst) = o;
+    tile_store<EPI>(a, grow, col, v, epb[EB ? k : 0], epr[ER ? k : 0]);
   }
   PI0_PROBE(3);
 }
 
-// ---- gated FFN on a wave grid, both operands staged in LDS ---------------------------
-// Workgroup = NW waves as (NW / 2) x 2: BM rows x 256 packed B columns (128 gate + the
-// matching 128 up), i.e. 128 output columns; wave (wm, wn) owns BM / (NW / 2) rows and
-// output columns wn * 64 .. + 64 (gate tiles 2 wn, 2 wn + 1 and the same up tiles). Per
-// 64-deep step a 384-row block loads 384 + 256 rows of 128 bytes for 384 x 256 x 64 MACs,
-// against 2 x (128 + 256) rows for 2 x 128 x 256 x 64 in the two-per-CU strip kernel
-// above, whose weight stream into VGPRs saturates the per-CU load path. Both operands go
-// global -> LDS directly (buffer_load ... lds, one 1 KB fragment per instruction) into a
-// D-slot ring of KS k16 slices per step, and every wave reads its A and B fragments from
-// there. One workgroup per CU (BM = 384, KS = 4: 80 KB per slot, two slots = all 160 KB
-// of LDS; 8 waves of 192 accumulators). Accumulation order per output element is the
-// strip kernel's (k16 fragments in k order), so the two kernels give bitwise-equal results.
-template <int BM, int D, int NW, int KS>
-__global__ __launch_bounds__(64 * NW, 1) void tile2_gated_kernel(TileArgs a) {
-  constexpr int WMR = NW / 2;              // wave rows (2 wave columns)
-  constexpr int FM = BM / (32 * WMR);      // 32-row fragments per wave
-  constexpr int FN = 4;                    // 2 gate + 2 up 32-column tiles per wave
-  constexpr int TA = (BM / 32) * KS;       // A fragments per step (KS k16 slices deep)
-  constexpr int TB = 8 * KS;               // B fragments per step (8 tiles x KS k16)
-  constexpr int CPW = NW / KS;             // tiles covered by one copy index
-  constexpr int LA = TA / NW, LB = TB / NW;  // ... issued by each wave
-  constexpr int SLOT = (TA + TB) * 64;     // 16-byte LDS words per ring slot
-  constexpr int OUTC = 128, OP = OUTC + 8; // output columns, bf16 pitch of the parked tile
-  constexpr int PARK = (BM * OP * 2 + 15) / 16;
-  static_assert(BM % (32 * WMR) == 0 && TA % NW == 0 && TB % NW == 0 && D >= 2, "tile shape");
-  static_assert(KS == 4 && NW % KS == 0 && 4 % CPW == 0, "copy assignment");
-  __shared__ bf16x8 lds[D * SLOT > PARK ? D * SLOT : PARK];
+// ---- 8-wave blocks, both operands staged in LDS ------------------------------------------
+// Workgroup = WMC x WNC waves over WMC FM 32 rows x WNC FN 32 packed B columns (DUAL: half of
+// them gate, half the matching up columns); wave (wm, wn) owns FM x FN fragments. Steps are
+// 32 deep in a ring of D slots (256 x 256: 32 KB each, three steps in flight while one is
+// multiplied). A instructions copy 16 rows x 64 bytes, B instructions one packed fragment.
+// Two things set the pace beside the MFMAs, and the loop is built around them:
+//   * the load path takes a copy in tens of clocks, so a burst of a step's copies blocks the
+//     waves that should be multiplying: half of a step's copies go out between the MFMAs of
+//     each k16 slice (256 x 256, K 2048: 87.5 -> 80.2k clocks, the MFMAs alone 65.5k);
+//   * a slice's fragments are read while the one before it is multiplied, into a second set
+//     of registers, across the step's barrier too: the barrier stands before the last slice,
+//     whose fragments are in registers, so it has MFMAs queued on both sides. Past it the
+//     step's slot is free for the step D - 1 ahead.
+// The k order of every accumulation is the strip kernel's: bitwise-equal products.
+template <int WMC, int WNC, int FM, int FN, int EPI, bool DUAL>
+__global__ __launch_bounds__(64 * WMC * WNC, 1) void block_gemm_kernel(TileArgs a) {
+  constexpr int D = 4, NW = WMC * WNC;
+  constexpr int BM = WMC * FM * 32, NBF = WNC * FN;      // rows, 32-column B fragments
+  constexpr int HT = DUAL ? NBF / 2 : NBF;               // B fragment columns per weight
+  constexpr int TA = BM / 16, TB = NBF * 2;              // copies of a step ...
+  constexpr int CC = (TA + TB + NW - 1) / NW, CH = CC / 2;   // ... per wave, in the last slice
+  // 16-byte LDS words: D slots of B, then D of A (fragment reads reach every B slot from one
+  // address register)
+  constexpr int SA = BM * 4, SB = NBF * 128, A0 = D * SB;
+  constexpr int OUTC = DUAL ? NBF * 16 : NBF * 32, CP = OUTC + 4, C8 = OUTC / 8;
+  constexpr int PR = WMC * 32;                           // rows parked per epilogue pass
+  constexpr int PARK = (PR * CP * 4 + 15) / 16;
+  constexpr int NEP = PR * C8 / (64 * NW);               // 8-column pieces per thread and pass
+  static_assert(!DUAL || FN % 2 == 0, "gate and up tiles of one wave");
+  static_assert(!DUAL || TA % NW == 0 || HT * 2 >= NW, "a mixed copy holds gate tiles only");
+  static_assert(FM * FN >= CC - CH, "a slice's copies between its MFMAs");
+  static_assert(NEP * 64 * NW == PR * C8 && BM % 16 == 0, "tile shape");
+  __shared__ bf16x8 lds[D * (SA + SB) > PARK ? D * (SA + SB) : PARK];
 
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  int id = blockIdx.x;
-  if (a.xcd_remap) id = (id & 7) * (gridDim.x >> 3) + (id >> 3);
-  const int mt = id % a.tiles_m, ntile = id / a.tiles_m;
-  const int m0 = mt * BM;
-  const int KT = a.K >> 4;
-  const int nsteps = a.ksteps;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wm = wave / WNC, wn = wave % WNC;
+  // XCD-contiguous tile order for any grid: workgroup b runs on XCD b % 8
+  int id;
+  {
+    const int b = blockIdx.x, x = b & 7, q = gridDim.x >> 3, r = gridDim.x & 7;
+    id = x * q + min(x, r) + (b >> 3);
+  }
+  const int mt = id % a.tiles_m;
+  id /= a.tiles_m;
+  const int ntile = id % a.tiles_n, ks = id / a.tiles_n;
+  const int m0 = mt * BM, KT = a.K >> 4, nsteps = a.ksteps, step0 = ks * a.ksteps;
 
   const int arows = max(min(BM, a.M - m0), 0);
   const __amdgpu_buffer_rsrc_t ar =
       rows_rsrc_sgpr(a.a + (size_t)m0 * a.lda, arows * a.lda * (int)sizeof(__bf16));
-  // gate tiles ntile * 4 + c and up tiles likewise; one resource per weight, starting at
-  // this block's first tile (its 4 tiles are contiguous: [nt][kt] order)
-  const int wbytes = 4 * KT * 512 * (int)sizeof(__bf16);
-  const __amdgpu_buffer_rsrc_t gr = rows_rsrc_sgpr(a.w0 + (size_t)ntile * 4 * KT * 512, wbytes);
-  const __amdgpu_buffer_rsrc_t ur = rows_rsrc_sgpr(a.w1 + (size_t)ntile * 4 * KT * 512, wbytes);
-  // copy q = i * NW + w of wave w is, of A, block rows 8 q .. 8 q + 7 (whole 128-byte step
-  // rows, chunks swizzled as in the strip kernel) and, of B, fragment q = tile * KS + slice
-  // (slice w % KS, tile i * CPW + w / KS); the i-dependent parts of the offsets are
-  // wave-uniform (scalar), so each operand needs one lane offset
-  const int avoff = ((wave * 8 + (lane >> 3)) * a.lda +
-                     ((lane & 7) ^ ((wave & 1) * 4 + (lane >> 4))) * 8) * (int)sizeof(__bf16);
-  const int afrag = (lane & 31) * 8 + ((lane >> 5) ^ ((lane >> 1) & 7));
   const int btile = KT * 512 * (int)sizeof(__bf16);
-  const int bvoff = ((wave % KS) * 512 + lane * 8) * (int)sizeof(__bf16) + (wave / KS) * btile;
-  const int arow_step = NW * 8 * a.lda * (int)sizeof(__bf16);
-
-  auto issue = [&](int s, int slot) {
-    const int abase = s * KS * 16 * (int)sizeof(__bf16);
-    const int bbase = s * KS * 512 * (int)sizeof(__bf16);
-    bf16x8* dst = lds + slot * SLOT;
-#pragma unroll
-    for (int i = 0; i < LA; ++i)
-      buf_load16_lds_s(ar, &dst[(i * NW + wave) * 64], avoff, abase + i * arow_step);
-#pragma unroll
-    for (int i = 0; i < LB; ++i)     // tiles 0-3 gate, 4-7 up
-      buf_load16_lds_s(i * CPW < 4 ? gr : ur, &dst[(TA + i * NW + wave) * 64], bvoff,
-                       bbase + ((i * CPW) & 3) * btile);
+  const __amdgpu_buffer_rsrc_t gr =
+      rows_rsrc_sgpr(a.w0 + (size_t)ntile * HT * KT * 512, HT * btile);
+  const __amdgpu_buffer_rsrc_t ur =
+      rows_rsrc_sgpr((DUAL ? a.w1 : a.w0) + (size_t)ntile * HT * KT * 512, HT * btile);
+  // A copy: row 16 q + lane / 4, LDS chunk lane % 4 of the row's four; chunk c of row r sits
+  // at c ^ (r / 4 % 4), so the fragment reads of 16 neighbouring rows hit distinct banks
+  const int avoff = ((lane >> 2) * a.lda + ((lane & 3) ^ (lane >> 4)) * 8) * (int)sizeof(__bf16);
+  const int afrag = (lane & 31) * 4 + ((lane >> 5) ^ ((lane >> 2) & 3));
+  const int bvoff = lane * 16, arow16 = 16 * a.lda * (int)sizeof(__bf16);
+  // copy i of this wave for step s: A rows first, then B fragments (tile q / 2, slice q % 2);
+  // a count that the waves do not divide repeats the last fragment
+  auto copy = [&](int s, int slot, int i) {
+    const int st = min(s, nsteps - 1) + step0;           // past the end: a harmless re-load
+    const int q = min(i * NW + wave, TA + TB - 1);
+    const int qb = q - TA, tile = qb >> 1;
+    const bool isa = q < TA, up = DUAL && tile >= HT;
+    const int soff = isa ? st * 64 + q * arow16
+                         : st * 2048 + (qb & 1) * 1024 + (up ? tile - HT : tile) * btile;
+    bf16x8* const da = &lds[A0 + slot * SA + q * 64];
+    bf16x8* const db = &lds[slot * SB + qb * 64];
+    if (i * NW + NW <= TA)
+      buf_load16_lds_s(ar, da, avoff, soff);
+    else if (i * NW >= TA)
+      buf_load16_lds_s(up ? ur : gr, db, bvoff, soff);
+    else                                                 // both kinds: B's first tiles
+      buf_load16_lds_s(isa ? ar : gr, isa ? da : db, isa ? avoff : bvoff, soff);
   };
 
   f32x16 acc[FM][FN];
@@ -425,65 +448,131 @@ __global__ __launch_bounds__(64 * NW, 1) void tile2_gated_kernel(TileArgs a) {
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  // fragment sets: A two, B two where the accumulators leave the registers for it; else B's
+  // next fragment follows each column's last MFMA into the same registers
+  constexpr bool B2 = FM * FN <= 10;
+  bf16x8 fa[2][FM], fb[B2 ? 2 : 1][FN];
+  auto read_a = [&](int slot, int kq, int b) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+      fa[b][i] = lds[A0 + slot * SA + (wm * FM + i) * 128 + (afrag ^ (kq * 2))];
+  };
+  auto read_b = [&](int slot, int kq, int b, int j) {
+    const int tile = DUAL ? (j < FN / 2 ? 0 : HT) + wn * (FN / 2) + j % (FN / 2) : wn * FN + j;
+    fb[B2 ? b : 0][j] = lds[slot * SB + (tile * 2 + kq) * 64 + lane];
+  };
+  // one slice: read the next one's fragments (slot rs, slice b ^ 1), multiply set b, with
+  // copies c0 .. c1 - 1 of step s spread between the MFMAs
+  auto slice = [&](int b, int rs, int s, int slot, int c0, int c1) {
+    constexpr int EV = FM * FN / (CC - CH) > 0 ? FM * FN / (CC - CH) : 1;
+    read_a(rs, b ^ 1, b ^ 1);
+    if constexpr (B2) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) read_b(rs, b ^ 1, b ^ 1, j);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int n = j * FM + i;
+        acc[i][j] = mfma32(fa[b][i], fb[B2 ? b : 0][j], acc[i][j]);
+        if (n % EV == EV / 2 && c0 + n / EV < c1) {
+          __builtin_amdgcn_sched_barrier(0);
+          copy(s, slot, c0 + n / EV);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      if constexpr (!B2) {
+        __builtin_amdgcn_sched_barrier(0);
+        read_b(rs, b ^ 1, 0, j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
 
 #pragma unroll
-  for (int u = 0; u < D - 1; ++u) issue(u, u);
-
+  for (int u = 0; u < D; ++u)
+#pragma unroll
+    for (int c = 0; c < (u < D - 1 ? CC : CH); ++c) copy(u, u, c);
+  __builtin_amdgcn_s_waitcnt(PI0_VMCNT((D - 2) * CC + CH));
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  read_a(0, 0, 0);
+#pragma unroll
+  for (int j = 0; j < FN; ++j) read_b(0, 0, 0, j);
   for (int s0 = 0; s0 < nsteps; s0 += D) {
 #pragma unroll
-    for (int u = 0; u < D; ++u) {
-      const int s = s0 + u;
-      // every copy of step s has landed (the D - 2 later steps may still be in flight)
-      __builtin_amdgcn_s_waitcnt(PI0_VMCNT((D - 2) * (LA + LB)));
+    for (int p = 0; p < D; ++p) {
+      const int s = s0 + p;
+      slice(0, p, s + D - 1, (p + D - 1) % D, CH, CC);   // the rest of that step's copies
+      // this wave's copies of step s + 1 have landed and its reads of step s are done; past
+      // the barrier the same holds for every wave
+      __builtin_amdgcn_s_waitcnt(PI0_VMCNT((D - 2) * CC) & ~(0xF << 8));
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      // past the end a harmless re-load of the last step keeps the count per step fixed
-      issue(min(s + D - 1, nsteps - 1), (u + D - 1) % D);
-      __builtin_amdgcn_sched_barrier(0);
-      const bf16x8* st = lds + u * SLOT;
-#pragma unroll
-      for (int kq = 0; kq < KS; ++kq) {
-        bf16x8 bf[FN];
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const int tile = (j < 2 ? 0 : 4) + wn * 2 + (j & 1);
-          bf[j] = st[(TA + tile * KS + kq) * 64 + lane];
-        }
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-          const bf16x8 af = st[(wm * FM + i) * 256 + (afrag ^ (kq * 2))];
-#pragma unroll
-          for (int j = 0; j < FN; ++j) acc[i][j] = mfma32(af, bf[j], acc[i][j]);
-        }
-        __builtin_amdgcn_sched_barrier(0);   // bound the fragments held: 384 accumulators
-      }
+      slice(1, (p + 1) % D, s + D, p, 0, CH);
     }
   }
 
-  // ---- epilogue: GeGLU in registers, parked as bf16 row-major, stored 16 bytes a lane
-  __builtin_amdgcn_s_waitcnt(PI0_VMCNT(0));
-  __syncthreads();
-  __bf16* cs = reinterpret_cast<__bf16*>(lds);
-  {
-    const int r = lane & 31, h = lane >> 5;
+  // ---- epilogue, FM passes of one row fragment of every wave: fp32 parked row-major, then 8
+  // columns of a row per thread with 16-byte loads and stores
+  __builtin_amdgcn_s_waitcnt(PI0_VMCNT(0));              // drain the harmless re-loads
+  constexpr bool EB = EPI == TE_BIAS || EPI == TE_BIAS_RES || EPI == TE_BIAS_GELU;
+  constexpr bool ER = EPI == TE_RES || EPI == TE_BIAS_RES;
+  const __amdgpu_buffer_rsrc_t br = rows_rsrc_sgpr(a.bias, EB ? a.n_valid * (int)sizeof(__bf16) : 0);
+  const int rrows = EPI == TE_RES ? a.M : (a.res_mod ? a.res_mod : a.M);
+  const int rld = EPI == TE_RES ? a.ldo : a.ldres;
+  const __amdgpu_buffer_rsrc_t rr =
+      rows_rsrc_sgpr(EPI == TE_RES ? (const void*)a.out : (const void*)a.res,
+                     ER ? rrows * rld * (int)sizeof(__bf16) : 0);
+  float* cs = reinterpret_cast<float*>(lds);
+  const int r = lane & 31, h = lane >> 5;
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+  for (int i = 0; i < FM; ++i) {
+    bf16x8 epb[EB ? NEP : 1], epr[ER ? NEP : 1];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int row = (wm * FM + i) * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          cs[row * OP + wn * 64 + j * 32 + r] = f2bf(gelu_tanh_rcp(acc[i][j][e]) * acc[i][2 + j][e]);
+    for (int k = 0; k < NEP; ++k) {
+      const int idx = t + 64 * NW * k, prow = idx / C8, col = ntile * OUTC + (idx - prow * C8) * 8;
+      const int grow = m0 + (prow >> 5) * (FM * 32) + i * 32 + (prow & 31);
+      if constexpr (EB) epb[k] = buf_load8(br, col * (int)sizeof(__bf16));
+      if constexpr (ER) {
+        const int rrow = EPI == TE_BIAS_RES && a.res_mod ? grow % a.res_mod : grow;
+        epr[k] = buf_load8(rr, rrow < rrows ? (rrow * rld + col) * (int)sizeof(__bf16) : INT_MAX - 64);
       }
-  }
-  __syncthreads();
-  constexpr int C8 = OUTC / 8;
-  for (int idx = t; idx < BM * C8; idx += 64 * NW) {
-    const int row = idx / C8, c = (idx - row * C8) * 8;
-    const int grow = m0 + row, col = ntile * OUTC + c;
-    if (grow >= a.M || col >= a.n_valid) continue;
-    *reinterpret_cast<bf16x8*>(a.out + (size_t)grow * a.ldo + col) =
-        *reinterpret_cast<const bf16x8*>(&cs[row * OP + c]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      float* row = cs + (wm * 32 + 8 * (e >> 2) + 4 * h + (e & 3)) * CP + r;
+      if constexpr (DUAL) {
+#pragma unroll
+        for (int j = 0; j < FN / 2; ++j)
+          row[(wn * (FN / 2) + j) * 32] = gelu_tanh_rcp(acc[i][j][e]) * acc[i][FN / 2 + j][e];
+      } else {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) row[(wn * FN + j) * 32] = acc[i][j][e];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NEP; ++k) {
+      const int idx = t + 64 * NW * k, prow = idx / C8, c = (idx - prow * C8) * 8;
+      const int grow = m0 + (prow >> 5) * (FM * 32) + i * 32 + (prow & 31);
+      const int col = ntile * OUTC + c;
+      if (grow >= a.M || col >= a.n_valid) continue;     // ragged rows, padded weight columns
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(&cs[prow * CP + c]);
+      const f32x4 hi = *reinterpret_cast<const f32x4*>(&cs[prow * CP + c + 4]);
+      if constexpr (EPI == TE_PARTIAL) {
+        float* dst = a.part + ((size_t)ks * a.M + grow) * a.N + col;
+        *reinterpret_cast<f32x4*>(dst) = lo;
+        *reinterpret_cast<f32x4*>(dst + 4) = hi;
+      } else {
+        float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        tile_store<EPI>(a, grow, col, v, epb[EB ? k : 0], epr[ER ? k : 0]);
+      }
+    }
   }
 }
 
@@ -510,17 +599,29 @@ __global__ void pack_weight32_kernel(const __bf16* __restrict__ w, __bf16* __res
   *reinterpret_cast<bf16x8*>(p + f * 8) = v;
 }
 
-// Split-K second pass: sum the partials in split order, add the residual, round once.
+// Split-K second pass: sum the partials in split order, add the residual, round once. The
+// split count is a compile-time one so that all partials of a piece are requested together
+// (0: any count).
+template <int S>
 __global__ __launch_bounds__(256) void tile_reduce_res_kernel(TileArgs a) {
   const int id = blockIdx.x * 256 + threadIdx.x;
   const int per_row = a.N >> 2;
   const int row = id / per_row, col = (id - row * per_row) * 4;
   if (row >= a.M) return;
-  f32x4 s = zero4();
-  for (int k = 0; k < a.splitk; ++k)
-    s += *reinterpret_cast<const f32x4*>(a.part + ((size_t)k * a.M + row) * a.N + col);
+  const float* src = a.part + (size_t)row * a.N + col;
+  const size_t stride = (size_t)a.M * a.N;
   __bf16* dst = a.out + (size_t)row * a.ldo + col;
   const bf16x4 rv = *reinterpret_cast<const bf16x4*>(dst);
+  f32x4 s = zero4();
+  if constexpr (S > 0) {
+    f32x4 p[S];
+#pragma unroll
+    for (int k = 0; k < S; ++k) p[k] = *reinterpret_cast<const f32x4*>(src + k * stride);
+#pragma unroll
+    for (int k = 0; k < S; ++k) s += p[k];
+  } else {
+    for (int k = 0; k < a.splitk; ++k) s += *reinterpret_cast<const f32x4*>(src + k * stride);
+  }
   const bf16x4 o = {f2bf(s[0] + bf2f(rv[0])), f2bf(s[1] + bf2f(rv[1])),
                     f2bf(s[2] + bf2f(rv[2])), f2bf(s[3] + bf2f(rv[3]))};
   *reinterpret_cast<bf16x4*>(dst) = o;
@@ -1064,22 +1165,39 @@ static int launch_tile_d4(TileArgs a, hipStream_t s) {
   return PI0HIP_ERR_SHAPE;
 }
 
-// Gated FFN on tile2_gated_kernel: BM-row x 128-output-column blocks, D-slot ring.
-template <int BM, int D, int NW, int KS>
-static int launch_tile2_gated(TileArgs a, hipStream_t s) {
-  const int kstep = KS * 16;
-  if (a.K % kstep || a.N % 128 || (a.K / kstep) % D) return PI0HIP_ERR_SHAPE;
-  if ((long long)a.K * 128 * (long long)sizeof(__bf16) > INT_MAX ||
+// block_gemm_kernel: K of a split a multiple of 4 steps of 32.
+template <int WMC, int WNC, int FM, int FN, int EPI, bool DUAL = false>
+static int launch_block(TileArgs a, hipStream_t s) {
+  constexpr int BM = WMC * FM * 32, NBF = WNC * FN, OUTC = DUAL ? NBF * 16 : NBF * 32;
+  if (a.splitk < 1 || a.K % (128 * a.splitk) || a.N % OUTC) return PI0HIP_ERR_SHAPE;
+  if ((long long)a.K * NBF * 32 * (long long)sizeof(__bf16) > INT_MAX ||
       (long long)BM * a.lda * (long long)sizeof(__bf16) > INT_MAX)
     return PI0HIP_ERR_SHAPE;                 // 32-bit buffer offsets
   a.tiles_m = (a.M + BM - 1) / BM;
-  a.tiles_n = a.N / 128;
-  a.splitk = 1;
-  a.ksteps = a.K / kstep;
-  const int grid = a.tiles_m * a.tiles_n;
-  a.xcd_remap = (grid % 8 == 0) ? 1 : 0;
-  hipLaunchKernelGGL((tile2_gated_kernel<BM, D, NW, KS>), dim3(grid), dim3(64 * NW), 0, s, a);
+  a.tiles_n = a.N / OUTC;
+  a.ksteps = a.K / 32 / a.splitk;
+  hipLaunchKernelGGL((block_gemm_kernel<WMC, WNC, FM, FN, EPI, DUAL>),
+                     dim3(a.tiles_m * a.tiles_n * a.splitk), dim3(64 * WMC * WNC), 0, s, a);
   return (int)hipGetLastError();
+}
+
+// Which tile a call takes. A launch of W workgroups runs in ceil(W / slots) rounds of about
+// equal length, so a tile whose grid just overflows a round loses up to half the chip: the
+// choice is the least rounds x (measured length of a full round). The lengths are single
+// launches with cold weights in a graph; what matters is their ratio, which K does not change
+// much. Kernels that share a CU (per_cu 2) refill it as they end, without rounds.
+static float tile_us(int M, int N, int bm, int bn, float round_us, int splitk = 1, int per_cu = 1) {
+  const float w = (float)((M + bm - 1) / bm) * (float)((N + bn - 1) / bn) * (float)splitk;
+  const float r = w / (float)(per_cu * device_cus());
+  return round_us * (per_cu > 1 ? fmaxf(r, 0.8f) : ceilf(r));
+}
+// ... of a block_gemm_kernel tile, which needs whole column tiles and 128-deep K
+static float block_us(int M, int N, int K, int bm, int bn, float round_us, int splitk = 1) {
+  if (N % bn || K % (128 * splitk)) return INFINITY;
+  return tile_us(M, N, bm, bn, round_us, splitk);
+}
+static int least(std::initializer_list<float> us) {
+  return (int)(std::min_element(us.begin(), us.end()) - us.begin());
 }
 
 static TileArgs tile_args(const void* x, int ldx, const void* w, void* out, int ldo, int M, int N,
@@ -1096,6 +1214,40 @@ static bool bad_dims(int M, int N, int K) { return M <= 0 || N <= 0 || K <= 0; }
 // 16-byte aligned (leading dimension a multiple of 8 bf16, pointer 16-byte aligned).
 static bool misaligned(const void* p, int ld) {
   return (reinterpret_cast<uintptr_t>(p) & 15) != 0 || (ld & 7) != 0;
+}
+
+// Plain and biased projections. Vision QKV (N = 3456, K = 1152), us before -> after: 256
+// rows 8.2 -> 6.5, 1024 13.8 -> 11.9, 2048 24.7 -> 21.2.
+template <int EPI>
+static int linear_launch(const TileArgs& a, hipStream_t s) {
+  const bool d3 = a.K % 192 == 0;
+  switch (least({tile_us(a.M, a.N, 64, 128, 8.5f), tile_us(a.M, a.N, 32, 128, 6.7f),
+                 d3 ? tile_us(a.M, a.N, 96, 128, 10.4f) : INFINITY,
+                 d3 ? tile_us(a.M, a.N, 96, 128, 21.2f, 1, 2) : INFINITY,
+                 block_us(a.M, a.N, a.K, 128, 128, 12.3f), block_us(a.M, a.N, a.K, 256, 128, 22.f)})) {
+    case 1: return launch_tile_d4<32, 32, EPI, false>(a, s);
+    case 2: case 3: return launch_tile<96, 32, 3, EPI, false, 2>(a, s);
+    case 4: return launch_block<4, 2, 1, 2, EPI>(a, s);
+    case 5: return launch_block<4, 2, 2, 2, EPI>(a, s);
+    default: return launch_tile_d4<64, 32, EPI, false>(a, s);
+  }
+}
+
+// Split-K partials of a residual GEMM (round lengths at 4096 of K per split).
+static int partial_launch(const TileArgs& a, hipStream_t s) {
+  // small M (the batched decoder, 204 rows): 32-row tiles, two workgroups per CU
+  if (a.M <= 256) return launch_tile_auto<32, 32, 4, TE_PARTIAL, false, 2>(a, s);
+  switch (least({tile_us(a.M, a.N, 192, 128, 57.f, a.splitk),
+                 block_us(a.M, a.N, a.K, 128, 256, 62.f, a.splitk),
+                 block_us(a.M, a.N, a.K, 192, 256, 92.f, a.splitk),
+                 block_us(a.M, a.N, a.K, 256, 256, 112.f, a.splitk),
+                 block_us(a.M, a.N, a.K, 384, 256, 155.f, a.splitk)})) {
+    case 1: return launch_block<2, 4, 2, 2, TE_PARTIAL>(a, s);
+    case 2: return launch_block<2, 4, 3, 2, TE_PARTIAL>(a, s);
+    case 3: return launch_block<4, 2, 2, 4, TE_PARTIAL>(a, s);
+    case 4: return launch_block<4, 2, 3, 4, TE_PARTIAL>(a, s);
+    default: return launch_tile_auto<192, 32, 4, TE_PARTIAL, false>(a, s);
+  }
 }
 
 extern "C" {
@@ -1138,16 +1290,7 @@ int pi0hip_tile_linear(const void* x, int ldx, const void* w_packed, const void*
   if (misaligned(x, ldx) || misaligned(out, ldo) || misaligned(bias, 0)) return PI0HIP_ERR_SHAPE;
   TileArgs a = tile_args(x, ldx, w_packed, out, ldo, M, N, K);
   a.bias = (const __bf16*)bias;
-  // 64-row tiles unless they overflow one round of the 256 CUs while 96-row tiles fit in
-  // one (vision QKV: 324 -> 216 workgroups at M = 768), or M is large (M >= 2048: the
-  // batched profile, where the taller tiles win by moving fewer bytes per flop).
-  const int steps = K / 64;
-  if (N % 128 == 0 && K % 64 == 0 && steps % 3 == 0 &&
-      ((((M + 63) / 64) * (N / 128) > 256 && ((M + 95) / 96) * (N / 128) <= 256) || M >= 2048))
-    return bias ? launch_tile<96, 32, 3, TE_BIAS, false, 2>(a, s)
-                : launch_tile<96, 32, 3, TE_STORE, false, 2>(a, s);
-  return bias ? launch_tile_d4<64, 32, TE_BIAS, false>(a, s)
-              : launch_tile_d4<64, 32, TE_STORE, false>(a, s);
+  return bias ? linear_launch<TE_BIAS>(a, s) : linear_launch<TE_STORE>(a, s);
 }
 
 int pi0hip_tile_linear_residual(const void* x, int ldx, const void* w_packed, void* out, int ldo,
@@ -1158,18 +1301,35 @@ int pi0hip_tile_linear_residual(const void* x, int ldx, const void* w_packed, vo
   TileArgs a = tile_args(x, ldx, w_packed, out, ldo, M, N, K);
   a.splitk = splitk;
   if (splitk == 1) {
-    // large M (>= 2048 rows): 128 x 256 tiles fill the chip without splitting K
-    if (M >= 2048 && N % 256 == 0) return launch_tile_d4<128, 64, TE_RES, false>(a, s);
-    return launch_tile_d4<64, 32, TE_RES, false>(a, s);
+    // o-proj (N = K = 2048), us before -> after: 1632 rows 23.2 -> 20.4, 2048 33.0 -> 21.6,
+    // 3264 36.5 -> 28.9, 4608 64.7 -> 43.6. A long K (ffn-down) keeps the 128 x 256 strip
+    // while that grid fits one round (3264 rows 217 us against 276 for the same block of
+    // block_gemm_kernel); past it 256 x 256 blocks, 6528 rows 475 -> 393.
+    if (K >= 8192 && M >= 2048 && N % 256 == 0) {
+      if (block_us(M, N, K, 256, 256, 393.f) < tile_us(M, N, 128, 256, 225.f))
+        return launch_block<4, 2, 2, 4, TE_RES>(a, s);
+      return launch_tile_d4<128, 64, TE_RES, false>(a, s);
+    }
+    switch (least({tile_us(M, N, 64, 128, 13.3f), block_us(M, N, K, 128, 128, 20.5f),
+                   block_us(M, N, K, 128, 256, 28.5f), block_us(M, N, K, 192, 256, 42.f),
+                   block_us(M, N, K, 256, 256, 56.f)})) {
+      case 1: return launch_block<4, 2, 1, 2, TE_RES>(a, s);
+      case 2: return launch_block<2, 4, 2, 2, TE_RES>(a, s);
+      case 3: return launch_block<2, 4, 3, 2, TE_RES>(a, s);
+      case 4: return launch_block<4, 2, 2, 4, TE_RES>(a, s);
+      default: return launch_tile_d4<64, 32, TE_RES, false>(a, s);
+    }
   }
   if (N % 4 || ldo % 4) return PI0HIP_ERR_SHAPE;
   if (!ws || ws_bytes < pi0hip_tile_workspace_bytes(M, N, splitk)) return PI0HIP_ERR_WORKSPACE;
   a.part = (float*)ws;
-  // small M (the batched decoder, 204 rows): 32-row tiles, two workgroups per CU
-  if (int e = M <= 256 ? launch_tile_auto<32, 32, 4, TE_PARTIAL, false, 2>(a, s)
-                       : launch_tile_auto<192, 32, 4, TE_PARTIAL, false>(a, s))
-    return e;
-  hipLaunchKernelGGL(tile_reduce_res_kernel, dim3((M * (N / 4) + 255) / 256), dim3(256), 0, s, a);
+  if (int e = partial_launch(a, s)) return e;
+  const dim3 rgrid((M * (N / 4) + 255) / 256);
+  switch (splitk) {
+    case 4: hipLaunchKernelGGL(tile_reduce_res_kernel<4>, rgrid, dim3(256), 0, s, a); break;
+    case 8: hipLaunchKernelGGL(tile_reduce_res_kernel<8>, rgrid, dim3(256), 0, s, a); break;
+    default: hipLaunchKernelGGL(tile_reduce_res_kernel<0>, rgrid, dim3(256), 0, s, a); break;
+  }
   return (int)hipGetLastError();
 }
 
@@ -1179,13 +1339,17 @@ int pi0hip_tile_gated_ffn(const void* x, int ldx, const void* gate_packed, const
   if (misaligned(x, ldx) || misaligned(out, ldo)) return PI0HIP_ERR_SHAPE;
   TileArgs a = tile_args(x, ldx, gate_packed, out, ldo, M, N, K);
   a.w1 = (const __bf16*)up_packed;
-  // From 512 rows (the prefix encoder: 768, batched 3264) the 8-wave 384-row blocks with
-  // both operands in LDS (768 rows: 115 -> 103 us with cold weights, bitwise equal); below,
-  // where 384-row blocks would be mostly padding, the two-per-CU strip kernel.
-  if (M >= 512) {
-    const int e = launch_tile2_gated<384, 2, 8, 4>(a, s);
-    if (e != PI0HIP_ERR_SHAPE) return e;
-  }
+  // Up to 256 rows the two-per-CU strip kernel's 128-row tiles (200 rows: 48 us against 54);
+  // above, blocks of 192, 256 or 384 rows x 128 outputs. us before -> after with the encoder's
+  // N = 16384, K = 2048: 269 rows 62.6 -> 48.1, 400 67 -> 59, 768 93 -> 89, 816 142 -> 108,
+  // 1024 148 -> 119, 3264 396 -> 380, 6528 771 -> 730.
+  if (M > 256 && N % 128 == 0 && K % 128 == 0)
+    switch (least({block_us(M, N, K, 192, 128, 50.f), block_us(M, N, K, 256, 128, 58.f),
+                   block_us(M, N, K, 384, 128, 86.f)})) {
+      case 0: return launch_block<2, 4, 3, 2, TE_GATE, true>(a, s);
+      case 1: return launch_block<4, 2, 2, 4, TE_GATE, true>(a, s);
+      default: return launch_block<4, 2, 3, 4, TE_GATE, true>(a, s);
+    }
   return launch_tile_auto<128, 64, 2, TE_GATE, true, 2>(a, s);
 }
 
@@ -1221,8 +1385,17 @@ int pi0hip_tile_qkv_rope_batched(const void* x, int ldx, const void* w_packed, c
   a.out_k = (__bf16*)k; a.out_v = (__bf16*)v; a.ldkv = ldkv;
   a.rope = (const __bf16*)rope; a.heads = heads; a.head_dim = head_dim;
   a.rows_per_batch = rows_per_batch; a.kv_bstride = kv_bstride;
-  if (M >= 2048 && a.N % 256 == 0) return launch_tile_d4<64, 64, TE_QKV_ROPE, false>(a, s);
-  return launch_tile_d4<64, 32, TE_QKV_ROPE, false>(a, s);
+  // us before -> after at N = 2560, K = 2048: 816 rows 24.3 -> 17.3 (260 workgroups of 64 x 128
+  // are two rounds), 1632 29.7 -> 24.8, 3264 53.4 -> 36.9, 6528 94 -> 67
+  switch (least({tile_us(M, a.N, 64, 128, 13.f), block_us(M, a.N, K, 128, 128, 18.f),
+                 block_us(M, a.N, K, 128, 256, 27.f), block_us(M, a.N, K, 192, 256, 38.f),
+                 block_us(M, a.N, K, 256, 256, 48.f)})) {
+    case 1: return launch_block<4, 2, 1, 2, TE_QKV_ROPE>(a, s);
+    case 2: return launch_block<2, 4, 2, 2, TE_QKV_ROPE>(a, s);
+    case 3: return launch_block<2, 4, 3, 2, TE_QKV_ROPE>(a, s);
+    case 4: return launch_block<4, 2, 2, 4, TE_QKV_ROPE>(a, s);
+    default: return launch_tile_d4<64, 32, TE_QKV_ROPE, false>(a, s);
+  }
 }
 
 int pi0hip_layer_norm(const void* x, int ldx, const void* w, const void* b, void* out, int ldo,
@@ -1294,13 +1467,18 @@ int pi0hip_tile_linear_bias_res(const void* x, int ldx, const void* w_packed, co
   a.bias = (const __bf16*)bias;
   a.res = (const __bf16*)res; a.ldres = ldres; a.res_mod = res_mod;
   // vision o-proj (K = 1152, 18 steps): a 3-deep ring, 7.1 us against 7.8-8.0 with 6 at
-  // M = 768, 17.3 against 19.2 at M = 3072
+  // M = 768, 17.3 against 19.2 at M = 3072. Rows per tile by the rounds they make (relative
+  // round lengths; o-proj at 1536 rows 11.5 -> 9.2 us, FFN-down 36.0 -> 34.2).
   const bool d3 = (K_pad / 64) % 3 == 0 && (K_pad / 64) % 4 != 0;
-  if (M >= 2048)
-    return d3 ? launch_tile<128, 32, 3, TE_BIAS_RES, false, 1>(a, s)
-              : launch_tile_auto<128, 32, 8, TE_BIAS_RES, false>(a, s);
-  return d3 ? launch_tile<32, 32, 3, TE_BIAS_RES, false, 1>(a, s)
-            : launch_tile_auto<32, 32, 8, TE_BIAS_RES, false>(a, s);
+  switch (least({tile_us(M, N_pad, 32, 128, 1.f), tile_us(M, N_pad, 64, 128, 1.42f),
+                 tile_us(M, N_pad, 128, 128, 2.05f)})) {
+    case 0: return d3 ? launch_tile<32, 32, 3, TE_BIAS_RES, false, 1>(a, s)
+                      : launch_tile_auto<32, 32, 8, TE_BIAS_RES, false>(a, s);
+    case 1: return d3 ? launch_tile<64, 32, 3, TE_BIAS_RES, false, 1>(a, s)
+                      : launch_tile_auto<64, 32, 8, TE_BIAS_RES, false>(a, s);
+    default: return d3 ? launch_tile<128, 32, 3, TE_BIAS_RES, false, 1>(a, s)
+                       : launch_tile_auto<128, 32, 8, TE_BIAS_RES, false>(a, s);
+  }
 }
 
 int pi0hip_tile_linear_bias_gelu(const void* x, int ldx, const void* w_packed, const void* bias,
@@ -1313,14 +1491,21 @@ int pi0hip_tile_linear_bias_gelu(const void* x, int ldx, const void* w_packed, c
   TileArgs a = tile_args(x, ldx, w_packed, out, ldo, M, N_pad, K_pad);
   a.n_valid = N;
   a.bias = (const __bf16*)bias;
-  // vision FFN up (K = 1152, N = 4352), two workgroups per CU: 128-column tiles at
-  // M = 768 (408 workgroups; 18.1 us against 18.7 with 256 columns), 256-column
-  // tiles from 2048 rows (M = 3072: 51 us against 58)
-  if (M < 2048 && N_pad % 128 == 0 && K_pad % 192 == 0)
-    return launch_tile<64, 32, 3, TE_BIAS_GELU, false, 2>(a, s);
-  if (N_pad % 256 == 0 && K_pad % 192 == 0)
-    return launch_tile<64, 64, 3, TE_BIAS_GELU, false, 2>(a, s);
-  return launch_tile_auto<64, 32, 8, TE_BIAS_GELU, false>(a, s);
+  // vision FFN up (K = 1152, N = 4352): 64 x 128 strips two to a CU while the grid is small
+  // (768 rows 16.3 us), then blocks by the rounds they make. us before -> after: 2048 rows
+  // 39.1 -> 32.2, 3072 50.3 -> 40.3, 4096 63.8 -> 55.7, 6144 86.6 -> 78.0.
+  const bool d3 = N_pad % 128 == 0 && K_pad % 192 == 0;
+  switch (least({d3 ? tile_us(M, N_pad, 64, 128, 17.f, 1, 2) : INFINITY,
+                 block_us(M, N_pad, K_pad, 128, 256, 26.5f), block_us(M, N_pad, K_pad, 192, 256, 33.f),
+                 block_us(M, N_pad, K_pad, 256, 256, 40.f), block_us(M, N_pad, K_pad, 384, 256, 56.f),
+                 1e30f})) {
+    case 0: return launch_tile<64, 32, 3, TE_BIAS_GELU, false, 2>(a, s);
+    case 1: return launch_block<2, 4, 2, 2, TE_BIAS_GELU>(a, s);
+    case 2: return launch_block<2, 4, 3, 2, TE_BIAS_GELU>(a, s);
+    case 3: return launch_block<4, 2, 2, 4, TE_BIAS_GELU>(a, s);
+    case 4: return launch_block<4, 2, 3, 4, TE_BIAS_GELU>(a, s);
+    default: return launch_tile_auto<64, 32, 8, TE_BIAS_GELU, false>(a, s);
+  }
 }
 
 int pi0hip_im2col_patches(const void* images, int views, void* out, int ldo, hipStream_t s) {

@@ -1,0 +1,105 @@
+"""The 8-wave block GEMMs at ragged row counts, one per tile that the dispatch can pick.
+
+Every tile accumulates each output over k in the same order, so a call's rows must be, bit for
+bit, those of the same entry called on at most 200 of them at a time (which the strip tiles
+serve; the oracle tests cover those). Sizes are one row into a tile's range or one short of
+its end; nothing may be stored past row M."""
+import pytest
+import torch
+
+from flash_vla_amd.backends.hip import _abi
+from flash_vla_amd.backends.hip import wrappers as W
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+CHUNK = 200
+
+
+def rnd(shape, seed, scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return (torch.randn(shape, generator=g, device=DEV) * scale).to(torch.bfloat16)
+
+
+def _rows_equal(M, N, call, init=None):
+    """call(row0, rows, out): the entry on rows row0 .. row0 + rows - 1, into `out`'s rows."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    whole = torch.full((M + 3, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    if init is not None:
+        whole[:M].copy_(init)
+    parts = whole.clone()
+    call(0, M, whole)
+    for r in range(0, M, CHUNK):
+        call(r, min(CHUNK, M - r), parts[r:])
+    torch.cuda.synchronize()
+    assert torch.isfinite(whole).all()
+    assert torch.equal(whole, parts)
+    assert torch.all(whole[M:] == 7.0), "stored past row M"
+
+
+@pytest.mark.parametrize("M", [257, 384, 385, 513, 768, 769, 1153])
+def test_gated_ffn_blocks(M):
+    K, N = 2048, 16384
+    x, g, u = rnd((M, K), 1), rnd((K, N), 2, 0.02), rnd((K, N), 3, 0.02)
+    gp, up = W.packed_weight_ptr(g, 32), W.packed_weight_ptr(u, 32)
+    _rows_equal(M, N, lambda r, n, out: _abi.call(
+        "pi0hip_tile_gated_ffn", x[r:].data_ptr(), K, gp, up, out.data_ptr(), N, n, N, K,
+        W._stream()))
+
+
+@pytest.mark.parametrize("M", [1025, 2049, 4097, 6201])
+def test_residual_blocks(M):
+    K, N = 2048, 2048
+    x, w, r0 = rnd((M, K), 4), rnd((K, N), 5, 0.02), rnd((M, N), 6)
+    wp = W.packed_weight_ptr(w, 32)
+    _rows_equal(M, N, lambda r, n, out: _abi.call(
+        "pi0hip_tile_linear_residual", x[r:].data_ptr(), K, wp, out.data_ptr(), N, n, N, K, 1,
+        None, 0, W._stream()), r0)
+
+
+@pytest.mark.parametrize("M,split", [(300, 8), (511, 8), (640, 8), (1001, 8), (1101, 4), (2047, 4),
+                                     (2305, 4)])
+def test_split_k_blocks(M, split):
+    K, N = 8192, 2048
+    x, w, r0 = rnd((M, K), 7), rnd((K, N), 8, 0.02), rnd((M, N), 9)
+    wp = W.packed_weight_ptr(w, 32)
+    ws = torch.empty(_abi.lib().pi0hip_tile_workspace_bytes(M, N, split), dtype=torch.uint8, device=DEV)
+    _rows_equal(M, N, lambda r, n, out: _abi.call(
+        "pi0hip_tile_linear_residual", x[r:].data_ptr(), K, wp, out.data_ptr(), N, n, N, K, split,
+        ws.data_ptr(), ws.numel(), W._stream()), r0)
+
+
+@pytest.mark.parametrize("M", [300, 993, 1153, 2047])
+def test_bias_blocks(M):
+    K, N = 1152, 3456
+    x, w, b = rnd((M, K), 10), rnd((K, N), 11, 0.03), rnd(N, 12, 0.5)
+    wp = W.packed_weight_ptr(w, 32)
+    _rows_equal(M, N, lambda r, n, out: _abi.call(
+        "pi0hip_tile_linear", x[r:].data_ptr(), K, wp, b.data_ptr(), out.data_ptr(), N, n, N, K,
+        W._stream()))
+
+
+@pytest.mark.parametrize("M", [1601, 1921, 2881, 4097])
+def test_bias_gelu_blocks(M):
+    K, N, N_pad = 1152, 4304, 4352
+    x, w, b = rnd((M, K), 13), rnd((K, N), 14, 0.03), rnd(N, 15, 0.5)
+    wp = W.packed_weight_ptr(w, 32, (K, N_pad))
+    _rows_equal(M, N, lambda r, n, out: _abi.call(
+        "pi0hip_tile_linear_bias_gelu", x[r:].data_ptr(), K, wp, b.data_ptr(), out.data_ptr(), N,
+        n, N, K, N_pad, K, W._stream()))
+
+
+@pytest.mark.parametrize("M", [769, 1601, 3201, 4801])
+def test_qkv_rope_blocks(M):
+    K, heads, hd = 2048, 8, 256
+    x, w, rope = rnd((M, K), 16), rnd((K, (heads + 2) * hd), 17, 0.02), rnd((M, hd), 18)
+    wp = W.packed_weight_ptr(w, 32)
+
+    def call(r, n, out):       # Q, K and V side by side in three of out's column ranges
+        q, k, v = (torch.full((n, c), 7.0, dtype=torch.bfloat16, device=DEV)
+                   for c in (heads * hd, hd, hd))
+        _abi.call("pi0hip_tile_qkv_rope", x[r:].data_ptr(), K, wp, rope[r:].data_ptr(),
+                  q.data_ptr(), k.data_ptr(), v.data_ptr(), hd, n, K, heads, hd, W._stream())
+        out[:n].copy_(torch.cat([q, k, v], 1))
+
+    _rows_equal(M, (heads + 2) * hd, call)
