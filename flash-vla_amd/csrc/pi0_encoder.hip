@@ -576,6 +576,116 @@ __global__ __launch_bounds__(64 * WMC * WNC, 1) void block_gemm_kernel(TileArgs 
   }
 }
 
+// ---- residual GEMM of a few hundred rows: 32 x 32 outputs over the whole K ----------------
+// out += x @ W for the batched decoder's o-proj and down (M = 204, N = 1024): as tiles of any
+// size these are too few to fill the chip without splitting K over workgroups, and the split
+// pays a second launch for its sum. Here the 8 waves of a workgroup split K and are summed
+// through LDS. What bounds it is the CU's load path, (32 + 32) K values per workgroup, so all
+// of it is asked for at once: each wave copies its x slice to LDS (whole 128-byte lines, four
+// 64-deep chunks, refilled in place once) and reads its packed W fragments into registers,
+// and multiplies a chunk as soon as the loads up to it have landed. The row blocks of a column
+// tile sit on one XCD, which then reads that weight tile from HBM once.
+template <int KT>     // k16 fragments per wave: K = 128 KT
+__global__ __launch_bounds__(512, 1) void rows32_res_kernel(TileArgs a, int nrb, int xcd_map) {
+  constexpr int NW = 8, NCH = KT / 4, SL = NCH < 4 ? NCH : 4;   // 64-deep chunks, LDS slots
+  static_assert(KT % 4 == 0 && NCH <= 2 * SL && 4 * SL + KT < 64, "chunks in flight");
+  __shared__ bf16x8 lds[NW * SL * 256];                        // 4 KB per chunk and wave
+  static_assert(sizeof(float) * NW * 1024 <= sizeof(lds), "reduction area");
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  int nt, rb;
+  if (xcd_map) {            // column tiles congruent to the XCD index, all row blocks each
+    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    nt = (j / nrb) * 8 + xcd;
+    rb = j - (j / nrb) * nrb;
+  } else {
+    nt = blockIdx.x / nrb;
+    rb = blockIdx.x - nt * nrb;
+  }
+  const int m0 = rb * 32, rows = min(32, a.M - m0);
+  const __amdgpu_buffer_rsrc_t xr =
+      rows_rsrc_sgpr(a.a + (size_t)m0 * a.lda, rows * a.lda * (int)sizeof(__bf16));
+  // the residual pair this thread finishes (row t / 16, columns 2 (t % 16) ..): first, so that
+  // every wait below covers it
+  const __amdgpu_buffer_rsrc_t orr =
+      rows_rsrc_sgpr(a.out + (size_t)m0 * a.ldo, rows * a.ldo * (int)sizeof(__bf16));
+  const int ooff = ((t >> 4) * a.ldo + nt * 32 + (t & 15) * 2) * (int)sizeof(__bf16);
+  const uint32_t res = __builtin_amdgcn_raw_buffer_load_b32(orr, ooff, 0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  // chunk copies: 8 rows x 128 bytes an instruction, 16-byte chunk c of row r at c ^ (r / 2 % 8)
+  bf16x8* const xs = lds + wave * SL * 256;
+  const int kw0 = wave * KT * 16;
+  const int xoff = ((lane >> 3) * a.lda + kw0) * (int)sizeof(__bf16);
+  auto copy = [&](int c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      buf_load16_lds_s(xr, xs + (c % SL) * 256 + i * 64,
+                       xoff + ((lane & 7) ^ ((i & 1) * 4 + (lane >> 4))) * 16,
+                       c * 128 + i * 8 * a.lda * (int)sizeof(__bf16));
+  };
+  const __bf16* wp = a.w0 + ((size_t)nt * (a.K >> 4) + wave * KT) * 512 + lane * 8;
+  bf16x8 bv[KT];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    if (c < SL) copy(c);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bv[c * 4 + i] = load8(wp + (c * 4 + i) * 512);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  f32x16 acc[2];            // even and odd fragments: two chains
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[0][e] = acc[1][e] = 0.f;
+  const int frag = (lane & 31) * 8 + ((lane >> 5) ^ ((lane >> 1) & 7));
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    // operations issued after chunk c's last: the later chunks' of the first pass, and the
+    // refills issued so far
+    constexpr int first = SL * 4 + KT;
+    const int pos = c < SL ? 8 * (c + 1) : first + 4 * (c - SL + 1);
+    const int issued = first + 4 * (NCH > SL ? min(c, NCH - SL) : 0);
+    __builtin_amdgcn_sched_barrier(0);
+    switch (issued - pos) {         // folds to one wait once the loop is unrolled
+#define PI0_W(n) case n: __builtin_amdgcn_s_waitcnt(PI0_VMCNT(n)); break;
+      PI0_W(0) PI0_W(4) PI0_W(8) PI0_W(12) PI0_W(16) PI0_W(20) PI0_W(24) PI0_W(28) PI0_W(32)
+      PI0_W(36) PI0_W(40) PI0_W(44)
+#undef PI0_W
+      default: __builtin_amdgcn_s_waitcnt(PI0_VMCNT(0)); break;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    bf16x8 av[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) av[i] = xs[(c % SL) * 256 + (frag ^ (i * 2))];
+    if (c + SL < NCH) {             // this wave's own slot: free once its reads are done
+      __builtin_amdgcn_s_waitcnt(0xC07F);                       // lgkmcnt(0)
+      __builtin_amdgcn_sched_barrier(0);
+      copy(c + SL);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i & 1] = mfma32(av[i], bv[c * 4 + i], acc[i & 1]);
+  }
+  __syncthreads();                  // every wave is done with its slice
+  float (*red)[16][PI0_WAVE] = reinterpret_cast<float (*)[16][PI0_WAVE]>(lds);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) red[wave][e][lane] = acc[0][e] + acc[1][e];
+  __syncthreads();
+  const int row = t >> 4, col = (t & 15) * 2;
+  if (row >= rows) return;
+  // C lane 32 h + col holds rows 8 (e / 4) + 4 h + e % 4
+  const int e = (row >> 3) * 4 + (row & 3), l = ((row >> 2) & 1) * 32 + col;
+  float v0 = 0.f, v1 = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    const float* p = &red[w][e][l];
+    v0 += p[0];
+    v1 += p[1];
+  }
+  const bf16x2 r2 = __builtin_bit_cast(bf16x2, res);
+  const bf16x2 o = {f2bf(v0 + bf2f(r2[0])), f2bf(v1 + bf2f(r2[1]))};
+  *reinterpret_cast<bf16x2*>(a.out + (size_t)(m0 + row) * a.ldo + nt * 32 + col) = o;
+}
+
 // W[batch][K][N] -> 32x32x16 B fragments: tile (nt, kt) of 16 k x 32 n is 64 lanes x 8 bf16,
 // lane = (k % 16 / 8) * 32 + n % 32, element k % 8; tiles ordered [nt][kt].
 // K_pad x N_pad (multiples of 16 / 32) with zeros outside the K x N source.
@@ -1181,6 +1291,17 @@ static int launch_block(TileArgs a, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
+static int launch_rows32(const TileArgs& a, hipStream_t s) {
+  const int nrb = (a.M + 31) / 32, ntiles = a.N / 32, xcd_map = ntiles % 8 == 0;
+  if (a.N % 32) return PI0HIP_ERR_SHAPE;
+  switch (a.K) {
+    case 2048: hipLaunchKernelGGL(rows32_res_kernel<16>, dim3(nrb * ntiles), dim3(512), 0, s, a, nrb, xcd_map); break;
+    case 4096: hipLaunchKernelGGL(rows32_res_kernel<32>, dim3(nrb * ntiles), dim3(512), 0, s, a, nrb, xcd_map); break;
+    default: return PI0HIP_ERR_SHAPE;
+  }
+  return (int)hipGetLastError();
+}
+
 // Which tile a call takes. A launch of W workgroups runs in ceil(W / slots) rounds of about
 // equal length, so a tile whose grid just overflows a round loses up to half the chip: the
 // choice is the least rounds x (measured length of a full round). The lengths are single
@@ -1310,13 +1431,20 @@ int pi0hip_tile_linear_residual(const void* x, int ldx, const void* w_packed, vo
         return launch_block<4, 2, 2, 4, TE_RES>(a, s);
       return launch_tile_d4<128, 64, TE_RES, false>(a, s);
     }
+    // The batched decoder's o-proj and down (N = 1024, K 2048 / 4096): 32 x 32 workgroups over
+    // the whole K, 204 rows 8.5 -> 4.9 and 11.2 -> 8.1 against 4 splits and their sum, 408
+    // rows 15.5 -> 8.1 and 20.8 -> 14.8.
+    const bool rows32 = (K == 2048 || K == 4096) && N % 32 == 0;
     switch (least({tile_us(M, N, 64, 128, 13.3f), block_us(M, N, K, 128, 128, 20.5f),
                    block_us(M, N, K, 128, 256, 28.5f), block_us(M, N, K, 192, 256, 42.f),
-                   block_us(M, N, K, 256, 256, 56.f)})) {
+                   block_us(M, N, K, 256, 256, 56.f), tile_us(M, N, 32, 128, 8.3f),
+                   rows32 ? tile_us(M, N, 32, 32, 5.2f) : INFINITY})) {
       case 1: return launch_block<4, 2, 1, 2, TE_RES>(a, s);
       case 2: return launch_block<2, 4, 2, 2, TE_RES>(a, s);
       case 3: return launch_block<2, 4, 3, 2, TE_RES>(a, s);
       case 4: return launch_block<4, 2, 2, 4, TE_RES>(a, s);
+      case 5: return launch_tile_d4<32, 32, TE_RES, false>(a, s);
+      case 6: return launch_rows32(a, s);
       default: return launch_tile_d4<64, 32, TE_RES, false>(a, s);
     }
   }

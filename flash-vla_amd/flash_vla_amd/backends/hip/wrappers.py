@@ -454,11 +454,13 @@ def _residual(x, weight, out, role):
                   _ptr(out), out.stride(0), M, N, K, _stream())
         return out
     if M > _TILE_M and K % 256 == 0 and N % 128 == 0:
-        s = 4
+        # the decoder's two K have a kernel that needs no split over workgroups
+        s = 1 if K in (2048, 4096) else 4
         nbytes = _abi.lib().pi0hip_tile_workspace_bytes(M, N, s)
-        ws = scratch(f"tile_ws_{role}", (nbytes,), torch.uint8, x.device)
+        ws = (scratch(f"tile_ws_{role}", (nbytes,), torch.uint8, x.device).data_ptr()
+              if nbytes else None)
         _abi.call("pi0hip_tile_linear_residual", _ptr(x), x.stride(0), packed_weight_ptr(weight, 32),
-                  _ptr(out), out.stride(0), M, N, K, s, ws.data_ptr(), nbytes, _stream())
+                  _ptr(out), out.stride(0), M, N, K, s, ws, nbytes, _stream())
         return out
     wp = packed_weight_ptr(weight)
     s = _splitk(M, N, K)

@@ -49,12 +49,32 @@ def test_gated_ffn_blocks(M):
 
 @pytest.mark.parametrize("M", [1025, 2049, 4097, 6201])
 def test_residual_blocks(M):
-    K, N = 2048, 2048
+    K, N = 3072, 2048      # not a K of the whole-K kernel, which sums in another order
     x, w, r0 = rnd((M, K), 4), rnd((K, N), 5, 0.02), rnd((M, N), 6)
     wp = W.packed_weight_ptr(w, 32)
     _rows_equal(M, N, lambda r, n, out: _abi.call(
         "pi0hip_tile_linear_residual", x[r:].data_ptr(), K, wp, out.data_ptr(), N, n, N, K, 1,
         None, 0, W._stream()), r0)
+
+
+@pytest.mark.parametrize("K", [2048, 4096])
+@pytest.mark.parametrize("M", [65, 96, 204, 257, 511])
+def test_whole_k_residual(M, K):
+    """32 x 32 outputs over the whole K, against a 64-bit product: bf16 rounding of the output
+    alone is 2^-9 of a value, the fp32 sums' order adds 1e-6 of the row's scale."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    N = 1024
+    x, w, r0 = rnd((M, K), 19), rnd((K, N), 20, 0.02), rnd((M, N), 21)
+    out = torch.full((M + 3, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    out[:M].copy_(r0)
+    _abi.call("pi0hip_tile_linear_residual", x.data_ptr(), K, W.packed_weight_ptr(w, 32),
+              out.data_ptr(), N, M, N, K, 1, None, 0, W._stream())
+    torch.cuda.synchronize()
+    ref = x.double() @ w.double() + r0.double()
+    tol = 2.0 ** -8 * ref.abs() + 1e-5 * ref.abs().max()
+    assert torch.all((out[:M].double() - ref).abs() <= tol)
+    assert torch.all(out[M:] == 7.0), "stored past row M"
 
 
 @pytest.mark.parametrize("M,split", [(300, 8), (511, 8), (640, 8), (1001, 8), (1101, 4), (2047, 4),
