@@ -370,6 +370,126 @@ __global__ __launch_bounds__(NW * 64, 1) void skinny_gemm_kernel(GemmArgs a) {
 }
 
 
+// QKV of a batch of requests (M = requests x rows > 64): 32 rows x NT column tiles of 16 per
+// workgroup. skinny_gemm_kernel gives each workgroup 64 rows x one tile, 640 workgroups of
+// 136 KB at M = 204 -- two and a half rounds of the chip, each bound by the CU's load path.
+// Here x is staged once for NT tiles: 224 workgroups of 224 KB at NT = 5, one round. Every
+// output's arithmetic is skinny_gemm_kernel's (the same fragments in the same order per wave,
+// the waves' sums and the squares joined in the same order), so a request's rows are bitwise
+// those of a batch of one. K = 1024 (8 k-tiles per wave). The weights go out first, as there.
+// Cold weights, M = 66: 7.9 -> 7.5 us, 204: 11.7 -> 7.7, 408: 18.0 -> 9.9.
+template <int NT>
+__global__ __launch_bounds__(256, 1) void qkv_rows32_kernel(GemmArgs a) {
+  constexpr int KTW = 8, NW = 4, KW = KTW * 32, NKB = 4, MT = 2, ROWS = 16 * MT;
+  constexpr int XIS = ROWS / 8;                   // x copies per 64-column k-block
+  static_assert(KTW * NT + NKB * XIS + NT < 64, "loads in flight");
+  constexpr size_t X_BYTES = (size_t)NW * ROWS * KW * 2;
+  constexpr size_t R_BYTES = ((size_t)NT * NW * MT * 4 * PI0_WAVE + NW * MT * PI0_WAVE) * 4;
+  __shared__ __attribute__((aligned(16))) char smem[X_BYTES > R_BYTES ? X_BYTES : R_BYTES];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int ct = blockIdx.x, m0 = blockIdx.y * ROWS, rows = min(ROWS, a.M - m0);
+  const int KT = a.K >> 5, kt0 = wave * KTW;
+  auto swz = [](int row) { return row & 7; };
+  __bf16* xs = reinterpret_cast<__bf16*>(smem) + wave * ROWS * KW;
+  // epilogue pieces: thread t finishes row (t / 4) % 32, columns 4 (t % 4).. of every other
+  // column tile; its RoPE entries are the oldest loads
+  constexpr int NP = (NT + 1) / 2;
+  const int lrow = (t >> 2) & (ROWS - 1), c4 = (t & 3) * 4, p0 = t >> 7;
+  bf16x4 rope4[NP];
+#pragma unroll
+  for (int j = 0; j < NP; ++j)
+    rope4[j] = qkv_rope_piece(a, m0 + lrow, ct * NT + min(p0 + 2 * j, NT - 1), c4);
+  __builtin_amdgcn_sched_barrier(0);
+  bf16x8 b[NT][KTW];
+#pragma unroll
+  for (int i = 0; i < KTW; ++i)
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+      b[n][i] = load8(a.w0 + ((size_t)(ct * NT + n) * KT + kt0 + i) * 512 + lane * 8);
+  __builtin_amdgcn_sched_barrier(0);
+  {
+    const __amdgpu_buffer_rsrc_t xr =
+        rows_rsrc_sgpr(a.x + (size_t)m0 * a.ldx, rows * a.ldx * (int)sizeof(__bf16));
+    const int row0 = lane >> 3, cl = lane & 7;
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb) {
+#pragma unroll
+      for (int q = 0; q < XIS; ++q) {
+        const int row = q * 8 + row0;
+        buf_load16_lds(xr, xs + kb * ROWS * 64 + q * 512,
+                       (row * a.ldx + (kt0 + kb * 2) * 32 + (cl ^ swz(row)) * 8) * (int)sizeof(__bf16));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  const int r = lane & 15, g = lane >> 4;
+  f32x4 acc[NT][MT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[n][mt] = zero4();
+  float ssl[MT] = {};
+#pragma unroll
+  for (int i = 0; i < KTW; ++i) {
+    if (i % 2 == 0) {       // every weight and the x copies up to k-block i / 2 have landed
+      __builtin_amdgcn_sched_barrier(0);
+      switch (i / 2) {
+        case 0: __builtin_amdgcn_s_waitcnt(PI0_VMCNT(3 * XIS)); break;
+        case 1: __builtin_amdgcn_s_waitcnt(PI0_VMCNT(2 * XIS)); break;
+        case 2: __builtin_amdgcn_s_waitcnt(PI0_VMCNT(XIS)); break;
+        default: __builtin_amdgcn_s_waitcnt(PI0_VMCNT(0)); break;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int xrow = mt * 16 + r;
+      const bf16x8 av = *reinterpret_cast<const bf16x8*>(
+          xs + (i / 2) * ROWS * 64 + xrow * 64 + (((i % 2) * 4 + g) ^ swz(xrow)) * 8);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) acc[n][mt] = mfma16(av, b[n][i], acc[n][mt]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bf16x2 q = {av[2 * j], av[2 * j + 1]};
+        ssl[mt] = __builtin_amdgcn_fdot2_f32_bf16(q, q, ssl[mt], false);
+      }
+    }
+  }
+  __syncthreads();                        // x staging area becomes the reduction area
+  typedef float RedT[NW][MT][4][PI0_WAVE];
+  RedT* red = reinterpret_cast<RedT*>(smem);
+  float (*ssred)[MT][PI0_WAVE] = reinterpret_cast<float (*)[MT][PI0_WAVE]>(smem + NT * sizeof(RedT));
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[n][wave][mt][i][lane] = acc[n][mt][i];
+    ssred[wave][mt][lane] = ssl[mt];
+  }
+  __syncthreads();
+  const int mt = lrow >> 4, r16 = lrow & 15, ii = r16 & 3, gg = r16 >> 2;
+  float ss = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ss += ssred[w][mt][q * 16 + r16];
+#pragma unroll
+  for (int j = 0; j < NP; ++j) {
+    const int n = p0 + 2 * j;
+    if (n >= NT) continue;
+    float v[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      float s0 = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) s0 += red[n][w][mt][ii][gg * 16 + c4 + c];
+      v[c] = s0;
+    }
+    gemm_epilogue<EPI_QKV_ROPE, false>(a, m0 + lrow, ct * NT + n, c4, (t & 3) == 0, v, v, ss, rope4[j]);
+  }
+}
+
 // Second pass of split-K: one workgroup per 64 x 16 output tile; thread t owns row
 // t/4, columns 4*(t%4)..; sums the splits in split order, then the epilogue. SK is the
 // split count when it is known at compile time (exactly SK partial loads), 0 for any
@@ -764,6 +884,12 @@ int pi0hip_norm_qkv_rope_batched(const void* x, int ldx, const void* wp, const v
   a.rope = (const __bf16*)rope; a.norm_factor = (__bf16*)norm_factor;
   a.heads = heads; a.head_dim = head_dim;
   a.batch = batch; a.kv_bstride = kv_bstride;
+  // from two 64-row blocks on, 32-row workgroups that share x between 5 column tiles
+  if (M > 64 && K == 1024 && (a.N / 16) % 5 == 0) {
+    if (bad_alignment(a)) return PI0HIP_ERR_SHAPE;
+    hipLaunchKernelGGL(qkv_rows32_kernel<5>, dim3(a.N / 80, (M + 31) / 32), dim3(256), 0, s, a);
+    return (int)hipGetLastError();
+  }
   return launch_gemm<EPI_QKV_ROPE, false>(a, s);
 }
 

@@ -123,3 +123,31 @@ def test_qkv_rope_blocks(M):
         out[:n].copy_(torch.cat([q, k, v], 1))
 
     _rows_equal(M, (heads + 2) * hd, call)
+
+
+@pytest.mark.parametrize("B,T", [(5, 13), (2, 33), (3, 41), (8, 64)])
+def test_batched_qkv_rows(B, T):
+    """The batch's 32-row workgroups against one request at a time (M = T <= 64), bit for bit."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    K, heads, hd = 1024, 8, 256
+    x, w, rope = rnd((B * T, K), 22), rnd((K, (heads + 2) * hd), 23, 0.02), rnd((T, hd), 24)
+
+    def run(xs, batch):
+        rows = xs.shape[0]
+        q = torch.zeros(rows * heads, hd, dtype=torch.bfloat16, device=DEV)
+        k = torch.zeros((batch, T + 1, hd), dtype=torch.bfloat16, device=DEV)
+        v, nf = k.clone(), torch.zeros(rows, dtype=torch.bfloat16, device=DEV)
+        args = (k[:, :T], v[:, :T]) if batch > 1 else (k[0, :T], v[0, :T])
+        W.decoder_norm_qkv_rope(xs, w, rope, q, *args, nf)
+        return q.view(batch, T, -1), k, v, nf
+
+    def row(b, t):           # states first
+        return b if t == 0 else B + b * (T - 1) + t - 1
+
+    q, k, v, nf = run(x, B)
+    for b in range(B):
+        idx = torch.tensor([row(b, t) for t in range(T)], device=DEV)
+        q1, k1, v1, nf1 = run(x[idx].contiguous(), 1)
+        assert torch.equal(q[b], q1[0]) and torch.equal(k[b], k1[0]) and torch.equal(v[b], v1[0])
+        assert torch.equal(nf[idx], nf1)
