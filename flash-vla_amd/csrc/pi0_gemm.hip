@@ -490,6 +490,136 @@ __global__ __launch_bounds__(256, 1) void qkv_rows32_kernel(GemmArgs a) {
   }
 }
 
+// Gated FFN of a small batch of requests (64 < M <= 256, K = 1024): one 16-column tile of gate
+// and up per workgroup, as for one request, with all rows streamed past it. The weights come
+// cold from HBM and are spread evenly this way (64 KB a CU; 32 x 128 tiles draw 512 KB a CU
+// and leave half the CUs idle at 102 rows); the rows are L2-resident. The 8 waves are 4 K
+// groups x 2 halves of the 32-row blocks; a wave keeps its 16 weight fragments in registers
+// and its x blocks pass through 16 KB of LDS in four 64-deep chunks, each refilled with the
+// next block's as soon as its fragments are read. Each output's arithmetic is
+// skinny_gemm_kernel's, so a request's rows are bitwise those of a batch of one. Each further
+// 64 rows cost a refill's round trip, 2 us, which is where the tiles take over. Cold weights,
+// us against the tiles: 66 rows 9.4 (13.1), 102 9.6 (13.2), 153 11.6 (13.4), 204 13.2 (13.4),
+// 306 19.2 (17.6).
+template <int NB>     // 32-row blocks per wave
+__global__ __launch_bounds__(512, 1) void gate_stream_kernel(GemmArgs a) {
+  constexpr int KTW = 8, NKG = 4, NCH = 4;
+  __shared__ bf16x8 lds[8 * NCH * 256];                   // [wave][chunk][32 rows][8 chunks]
+  __shared__ float ssred[NKG][2 * NB][2][PI0_WAVE];
+  typedef float RedT[2 * NB][2][2][4][PI0_WAVE];          // [block][mt][gate, up][i][lane]
+  static_assert(NKG * sizeof(RedT) <= sizeof(lds), "reduction area");
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), kg = wave >> 1, rh = wave & 1;
+  const int nt = blockIdx.x, KT = a.K >> 5, kt0 = kg * KTW;
+  bf16x8 b0[KTW], b1[KTW];
+  {
+    const size_t o = ((size_t)nt * KT + kt0) * 512 + lane * 8;
+#pragma unroll
+    for (int i = 0; i < KTW; ++i) {
+      b0[i] = load8(a.w0 + o + i * 512);
+      b1[i] = load8(a.w1 + o + i * 512);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // x copies: chunk c of row block j of this wave (block 2 j + rh), 8 rows x 128 bytes an
+  // instruction; 16-byte chunk q of row r at q ^ (r / 2 % 8). Rows past M read as zeros.
+  const __amdgpu_buffer_rsrc_t xr = rows_rsrc_sgpr(a.x, a.M * a.ldx * (int)sizeof(__bf16));
+  bf16x8* const xs = lds + wave * NCH * 256;
+  const int xoff = ((lane >> 3) * a.ldx + kt0 * 32) * (int)sizeof(__bf16);
+  auto copy = [&](int j, int c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      buf_load16_lds_s(xr, xs + c * 256 + i * 64,
+                       xoff + ((lane & 7) ^ ((i & 1) * 4 + (lane >> 4))) * 16,
+                       c * 128 + ((2 * j + rh) * 32 + i * 8) * a.ldx * (int)sizeof(__bf16));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) copy(0, c);
+  const int r = lane & 15, g = lane >> 4;
+  f32x4 acc[NB][2][2];
+  float ssl[NB][2];
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      acc[j][mt][0] = acc[j][mt][1] = zero4();
+      ssl[j][mt] = 0.f;
+    }
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      // copies issued after this chunk's: the other three chunks' (this block's or the next's)
+      __builtin_amdgcn_sched_barrier(0);
+      if (j < NB - 1 || c == 0) __builtin_amdgcn_s_waitcnt(PI0_VMCNT(12));
+      else if (c == 1) __builtin_amdgcn_s_waitcnt(PI0_VMCNT(8));
+      else if (c == 2) __builtin_amdgcn_s_waitcnt(PI0_VMCNT(4));
+      else __builtin_amdgcn_s_waitcnt(PI0_VMCNT(0));
+      __builtin_amdgcn_sched_barrier(0);
+      bf16x8 av[2][2];                                    // [k-tile][mt]
+#pragma unroll
+      for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+          const int row = mt * 16 + r;
+          av[k2][mt] = xs[c * 256 + row * 8 + ((k2 * 4 + g) ^ ((row >> 1) & 7))];
+        }
+      if (j < NB - 1) {                                   // this wave's own chunk: read, refill
+        __builtin_amdgcn_s_waitcnt(0xC07F);               // lgkmcnt(0)
+        __builtin_amdgcn_sched_barrier(0);
+        copy(j + 1, c);
+      }
+#pragma unroll
+      for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+          acc[j][mt][0] = mfma16(av[k2][mt], b0[c * 2 + k2], acc[j][mt][0]);
+          acc[j][mt][1] = mfma16(av[k2][mt], b1[c * 2 + k2], acc[j][mt][1]);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const bf16x2 s2 = {av[k2][mt][2 * q], av[k2][mt][2 * q + 1]};
+            ssl[j][mt] = __builtin_amdgcn_fdot2_f32_bf16(s2, s2, ssl[j][mt], false);
+          }
+        }
+    }
+  __syncthreads();                                        // the x chunks become the sums' area
+  RedT* red = reinterpret_cast<RedT*>(lds);
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        red[kg][2 * j + rh][mt][0][i][lane] = acc[j][mt][0][i];
+        red[kg][2 * j + rh][mt][1][i][lane] = acc[j][mt][1][i];
+      }
+      ssred[kg][2 * j + rh][mt][lane] = ssl[j][mt];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < (NB + 1) / 2; ++p) {                // 4-column pieces, 4 to a row
+    const int id = t + 512 * p, row = id >> 2, c4 = (id & 3) * 4;
+    if (row >= min(a.M, 64 * NB)) continue;
+    const int bl = row >> 5, mt = (row >> 4) & 1, r16 = row & 15, ii = r16 & 3, gg = r16 >> 2;
+    float v0[4], v1[4], ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      v0[c] = v1[c] = 0.f;
+#pragma unroll
+      for (int k = 0; k < NKG; ++k) {
+        v0[c] += red[k][bl][mt][0][ii][gg * 16 + c4 + c];
+        v1[c] += red[k][bl][mt][1][ii][gg * 16 + c4 + c];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NKG; ++k)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) ss += ssred[k][bl][mt][q * 16 + r16];
+    gemm_epilogue<EPI_GATE, true>(a, row, nt, c4, false, v0, v1, ss);
+  }
+}
+
 // Second pass of split-K: one workgroup per 64 x 16 output tile; thread t owns row
 // t/4, columns 4*(t%4)..; sums the splits in split order, then the epilogue. SK is the
 // split count when it is known at compile time (exactly SK partial loads), 0 for any
@@ -949,6 +1079,14 @@ int pi0hip_norm_gated_ffn(const void* x, int ldx, const void* gate_p, const void
   if (!x || !gate_p || !up_p || !out) return PI0HIP_ERR_ARG;
   GemmArgs a = base_args(x, ldx, gate_p, out, ldo, M, N, K, 1);
   a.w1 = (const __bf16*)up_p;
+  if (M > 64 && M <= 256 && K == 1024 && N > 0 && N % 16 == 0) {
+    if (bad_alignment(a)) return PI0HIP_ERR_SHAPE;
+    const dim3 grid(N / 16), block(512);
+    if (M <= 128) hipLaunchKernelGGL(gate_stream_kernel<2>, grid, block, 0, s, a);
+    else if (M <= 192) hipLaunchKernelGGL(gate_stream_kernel<3>, grid, block, 0, s, a);
+    else hipLaunchKernelGGL(gate_stream_kernel<4>, grid, block, 0, s, a);
+    return (int)hipGetLastError();
+  }
   return launch_gemm<EPI_GATE, true>(a, s);
 }
 

@@ -486,7 +486,9 @@ def _gated_ffn(x, gate_w, up_w, out):
     N = gate_w.shape[1]
     if gate_w.shape != (K, N) or up_w.shape != (K, N) or out.shape != (M, N):
         raise ValueError("decoder_norm_gated_ffn: shape mismatch")
-    if M > _TILE_M and K % 128 == 0 and N % 128 == 0:
+    # up to 256 rows of the decoder's width the one-request layout, rows streamed past it
+    stream = K == 1024 and M <= 256
+    if M > _TILE_M and not stream and K % 128 == 0 and N % 128 == 0:
         _abi.call("pi0hip_tile_norm_gated_ffn", _ptr(x), x.stride(0), packed_weight_ptr(gate_w, 32),
                   packed_weight_ptr(up_w, 32), _ptr(out), out.stride(0), M, N, K, _stream())
         return out

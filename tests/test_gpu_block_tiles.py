@@ -151,3 +151,20 @@ def test_batched_qkv_rows(B, T):
         q1, k1, v1, nf1 = run(x[idx].contiguous(), 1)
         assert torch.equal(q[b], q1[0]) and torch.equal(k[b], k1[0]) and torch.equal(v[b], v1[0])
         assert torch.equal(nf[idx], nf1)
+
+
+@pytest.mark.parametrize("M", [65, 128, 129, 192, 193, 256])
+def test_batched_gate_rows(M):
+    """All rows of a batch streamed past a column tile, against 64 rows at a time, bit for bit."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    K, N = 1024, 4096
+    x, g, u = rnd((M, K), 25), rnd((K, N), 26, 0.02), rnd((K, N), 27, 0.02)
+    out = torch.full((M + 3, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    W.decoder_norm_gated_ffn(x, g, u, out[:M], None)
+    for r in range(0, M, 64):
+        n = min(64, M - r)
+        part = torch.zeros(n, N, dtype=torch.bfloat16, device=DEV)
+        W.decoder_norm_gated_ffn(x[r:r + n], g, u, part, None)
+        assert torch.equal(out[r:r + n], part)
+    assert torch.all(out[M:] == 7.0), "stored past row M"
