@@ -1067,131 +1067,139 @@ __global__ __launch_bounds__(256) void im2col_patches_kernel(const __bf16* __res
 }
 
 // Multi-head vision attention (attention.py:20-26, SDPA over each view's 256 tokens,
-// 16 heads of 72). V of every (view, head) is first transposed into
-// vt[view][head][96 d][tokens] (d >= 72 zero; keys of every 16-key chunk in the P^T
-// slot order, as for the encoder), then one wave per (view, head, 32 queries) runs
-// S^T = K Q^T / O^T = V^T P^T on 32x32x16 MFMAs over the 8 key blocks (head_dim
-// zero-padded to 80 for the k16 steps), softmax in fp32 with P rounded to bf16.
-constexpr int VA_TOK = 256, VA_HD = 72, VA_HDP = 96;
-
-__global__ __launch_bounds__(256) void vision_vt_kernel(const __bf16* __restrict__ qkv, int ldqkv,
-                                                        __bf16* __restrict__ vt, int heads,
-                                                        int dim) {
-  __shared__ __attribute__((aligned(16))) __bf16 tile[64][VA_HD + 8];
-  const int kc = blockIdx.x, head = blockIdx.y, view = blockIdx.z;
-  const int t = threadIdx.x;
-  const __bf16* src = qkv + ((size_t)view * VA_TOK + kc * 64) * ldqkv + 2 * dim + head * VA_HD;
-  // 16-byte loads: 64 key rows x 9 chunks of 8 head dims
-  for (int i = t; i < 64 * 9; i += 256) {
-    const int kr = i / 9, c = (i - kr * 9) * 8;
-    *reinterpret_cast<bf16x8*>(&tile[kr][c]) = load8(src + (size_t)kr * ldqkv + c);
-  }
-  __syncthreads();
-  // 16-byte stores: 96 padded dims x 8 chunks of 8 storage slots (keys in P^T slot order)
-  __bf16* dst = vt + (((size_t)view * heads + head) * VA_HDP) * VA_TOK + kc * 64;
-  for (int i = t; i < VA_HDP * 8; i += 256) {
-    const int d = i >> 3, c = (i & 7) * 8;
-    bf16x8 o;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int slot = c + q, sl = slot & 15;
-      const int key = (slot & ~15) + ((sl & 4) ? 8 : 0) + ((sl & 8) ? 4 : 0) + (sl & 3);
-      o[q] = d < VA_HD ? tile[key][d] : __bf16(0.f);
-    }
-    *reinterpret_cast<bf16x8*>(dst + (size_t)d * VA_TOK + c) = o;
-  }
-}
+// 16 heads of 72). A workgroup stages one (view, head)'s K and V in LDS straight from the
+// packed QKV rows (buffer loads with the LDS destination, rows of 144 bytes: nine 16-byte
+// chunks, an odd count, so the fragment reads of 16 neighbouring rows hit distinct banks) and
+// takes 2 tiles of 32 queries, each over 2 halves of the keys: wave = (query tile, key half).
+// S^T = K Q^T and O^T = V^T P^T on 32x32x16 MFMAs (head_dim zero-padded to 80 for the k16
+// steps), softmax in fp32 with P rounded to bf16 and normalised by the rounded P's sum. All of
+// a wave's scores are held at once, so there is one maximum and no rescaling. V^T comes from row-major V by transposing LDS reads:
+// within a 16-lane group lane 4 k + c points at 4 columns of key k and lane j receives 4 keys
+// of column j, which is half of an A fragment in the key order that P^T has in the S^T
+// accumulator. A launch that transposed V through memory, waves reading both from L2 and an
+// online softmax took 13.8 us at 3 views and 35.9 at 12; this takes 6.6 and 21.5, at the same
+// distance from 64 bits (2.15e-3). One 4-tile workgroup over all keys: 7.2 and 20.6, but
+// 2.19e-3 (a maximum over more keys leaves fewer P that are exactly 1).
+constexpr int VA_TOK = 256, VA_HD = 72;
 
 struct VisAttnArgs {
   const __bf16* qkv; int ldqkv;
-  const __bf16* vt;
   __bf16* out; int ldo;
-  int heads, dim;
+  int dim;
   float scale_log2;
 };
 
-// One wave per 32 queries of a (view, head); a workgroup holds NWQ consecutive query tiles
-// of the same (view, head), whose waves read the same K / V^T fragments.
-template <int NWQ>
-__global__ __launch_bounds__(64 * NWQ, 1) void vision_attn_kernel(VisAttnArgs a) {
+constexpr int VA_QT = 2, VA_KS = 2;                     // query tiles, key parts per workgroup
+
+__global__ __launch_bounds__(64 * VA_QT * VA_KS, 1) void vision_attn_kernel(VisAttnArgs a) {
+  constexpr int QT = VA_QT, KS = VA_KS, NW = QT * KS, CH = VA_HD / 8, WORDS = VA_TOK * CH, CI = WORDS / (64 * NW);
+  constexpr int NB = VA_TOK / 32 / KS;                  // 32-key blocks of a wave
+  static_assert(CI * 64 * NW == WORDS && NB * 32 * KS == VA_TOK, "staging and key split");
+  // K, then V; the padded head dims of V's last rows are read (and not used) past the end
+  __shared__ bf16x8 kv[2 * WORDS + 32];
   PI0_PROBE(0);
-  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
-  const int qt = blockIdx.x * NWQ + (threadIdx.x >> 6), head = blockIdx.y, view = blockIdx.z;
-  const size_t row0 = (size_t)view * VA_TOK;
-  const int q = qt * 32 + r;
+  const int t = threadIdx.x, lane = t & 63, r = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), qi = wave / KS, kp = wave % KS;
+  const int head = blockIdx.y, view = blockIdx.z;
+  const __bf16* base = a.qkv + (size_t)view * VA_TOK * a.ldqkv + head * VA_HD;
+  const int nbytes = ((VA_TOK - 1) * a.ldqkv + VA_HD) * (int)sizeof(__bf16);
+  const __amdgpu_buffer_rsrc_t kr = rows_rsrc_sgpr(base + a.dim, nbytes);
+  const __amdgpu_buffer_rsrc_t vr = rows_rsrc_sgpr(base + 2 * a.dim, nbytes);
+  int off[CI];
+#pragma unroll
+  for (int i = 0; i < CI; ++i) {
+    const int id = (i * NW + wave) * 64 + lane, row = id / CH;
+    off[i] = (row * a.ldqkv + (id - row * CH) * 8) * (int)sizeof(__bf16);
+    buf_load16_lds(kr, &kv[(i * NW + wave) * 64], off[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < CI; ++i) buf_load16_lds(vr, &kv[WORDS + (i * NW + wave) * 64], off[i]);
+  __builtin_amdgcn_sched_barrier(0);
   // Q^T fragments: lane holds Q[q][16 kk + 8 h .. + 7] (zero past d = 72)
+  const int q = (blockIdx.x * QT + qi) * 32 + r;
   bf16x8 qf[5];
 #pragma unroll
   for (int kk = 0; kk < 5; ++kk) {
     const int d = kk * 16 + h * 8;
-    qf[kk] = d < VA_HD ? load8(a.qkv + (row0 + q) * a.ldqkv + head * VA_HD + d) : zero8();
+    qf[kk] = d < VA_HD ? load8(base + (size_t)q * a.ldqkv + d) : zero8();
   }
-  float m_run = -1.0e30f, l_run = 0.f;
+  f32x16 st[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) st[b][e] = 0.f;
+  __syncthreads();                                      // waits for every copy
+  PI0_PROBE(1);
+  const int key0 = kp * NB * 32;
+#pragma unroll
+  for (int kk = 0; kk < 5; ++kk)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      bf16x8 kf = kv[(key0 + b * 32 + r) * CH + kk * 2 + (kk < 4 ? h : 0)];
+      if (kk == 4 && h) kf = zero8();                   // head dims 72 .. 79
+      st[b] = mfma32(kf, qf[kk], st[b]);
+    }
+  // lane holds S^T[key 32 b + 8 (e / 4) + 4 h + e % 4][query r]
+  float mx = -1.0e30f, l = 0.f;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) { st[b][e] *= a.scale_log2; mx = fmaxf(mx, st[b][e]); }
+  mx = fmaxf(mx, __shfl_xor(mx, 32, PI0_WAVE));
   f32x16 o[3];
 #pragma unroll
   for (int dt = 0; dt < 3; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
-  const __bf16* vt = a.vt + (((size_t)view * a.heads + head) * VA_HDP) * VA_TOK;
-  // A three-slot register ring over the 8 key blocks: block kb + 3 is requested as soon
-  // as block kb has consumed its slot, so two blocks are always in flight.
-  constexpr int NB = VA_TOK / 32, RS = 3;
-  bf16x8 kf[RS][5], vf[RS][3][2];
-  auto load_blk = [&](int kb) {
-    const int sl = kb % RS;
-    // columns 72..79 of the padded head are read unmasked (the next head's K, or for the
-    // last head the first V columns of the same row): Q^T is zero there, so they add 0
+  typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+  const __bf16* vs = reinterpret_cast<const __bf16*>(kv + WORDS);
+  const int vlane = (key0 + 4 * h + ((lane & 15) >> 2)) * VA_HD + (lane & 16) + (lane & 3) * 4;
 #pragma unroll
-    for (int kk = 0; kk < 5; ++kk)
-      kf[sl][kk] = load8(a.qkv + (row0 + kb * 32 + r) * a.ldqkv + a.dim + head * VA_HD + kk * 16 + h * 8);
+  for (int b = 0; b < NB; ++b) {
+    bf16x8 pf[2];                                       // P^T for chunk c = e / 8
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      pf[e >> 3][e & 7] = f2bf(fast_exp2(st[b][e] - mx));
+      l += bf2f(pf[e >> 3][e & 7]);
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int dt = 0; dt < 3; ++dt) {
+        const int at = vlane + (b * 32 + c * 16) * VA_HD + dt * 32;
+        const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(vs + at));
+        const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(vs + at + 8 * VA_HD));
+        const bf16x8 vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        o[dt] = mfma32(vf, pf[c], o[dt]);
+      }
+  }
+  l += __shfl_xor(l, 32, PI0_WAVE);
+  PI0_PROBE(2);
+  {                                                     // join the key halves
+    static_assert(KS == 2, "one part parked per query tile");
+    float* park = reinterpret_cast<float*>(kv) + qi * 50 * PI0_WAVE + lane;
+    __syncthreads();                                    // every wave is done with K and V
+    if (kp == 1) {
+      park[0] = mx;
+      park[PI0_WAVE] = l;
+#pragma unroll
+      for (int dt = 0; dt < 3; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) park[(2 + dt * 16 + e) * PI0_WAVE] = o[dt][e];
+    }
+    __syncthreads();
+    if (kp == 1) return;
+    const float m1 = park[0], m = fmaxf(mx, m1);
+    const float w0 = fast_exp2(mx - m), w1 = fast_exp2(m1 - m);
+    l = l * w0 + park[PI0_WAVE] * w1;
 #pragma unroll
     for (int dt = 0; dt < 3; ++dt)
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
-        vf[sl][dt][c] = load8(vt + (size_t)(dt * 32 + r) * VA_TOK + kb * 32 + 16 * c + 8 * h);
-  };
-#pragma unroll
-  for (int kb = 0; kb < RS; ++kb) load_blk(kb);
-#pragma unroll
-  for (int kb = 0; kb < NB; ++kb) {
-    const int sl = kb % RS;
-    PI0_PROBE(8 + kb);
-    f32x16 st;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) st[e] = 0.f;
-#pragma unroll
-    for (int kk = 0; kk < 5; ++kk) st = mfma32(kf[sl][kk], qf[kk], st);
-    float mx = -1.0e30f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) { st[e] *= a.scale_log2; mx = fmaxf(mx, st[e]); }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, PI0_WAVE));
-    const float m_new = fmaxf(m_run, mx);
-    const float alpha = fast_exp2(m_run - m_new);
-    float ps = 0.f;
-    bf16x8 pf[2];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const float pv = fast_exp2(st[e] - m_new);
-      ps += pv;
-      pf[e >> 3][e & 7] = f2bf(pv);
-    }
-    ps += __shfl_xor(ps, 32, PI0_WAVE);
-    l_run = l_run * alpha + ps;
-    m_run = m_new;
-#pragma unroll
-    for (int dt = 0; dt < 3; ++dt) {
-      f32x16 acc = o[dt] * alpha;
-#pragma unroll
-      for (int c = 0; c < 2; ++c) acc = mfma32(vf[sl][dt][c], pf[c], acc);
-      o[dt] = acc;
-    }
-    if (kb + RS < NB) load_blk(kb + RS);
-    __builtin_amdgcn_sched_barrier(0);                 // keep each refill in its iteration
+      for (int e = 0; e < 16; ++e) o[dt][e] = o[dt][e] * w0 + park[(2 + dt * 16 + e) * PI0_WAVE] * w1;
   }
-  PI0_PROBE(2);
   // lane holds O^T[d = 32 dt + 8 (e / 4) + 4 h + e % 4][query r]
-  const float inv = __builtin_amdgcn_rcpf(l_run);
-  __bf16* orow = a.out + (row0 + q) * a.ldo + head * VA_HD;
+  const float inv = __builtin_amdgcn_rcpf(l);
+  __bf16* orow = a.out + ((size_t)view * VA_TOK + q) * a.ldo + head * VA_HD;
 #pragma unroll
   for (int dt = 0; dt < 3; ++dt)
 #pragma unroll
@@ -1646,34 +1654,23 @@ int pi0hip_im2col_patches(const void* images, int views, void* out, int ldo, hip
   return (int)hipGetLastError();
 }
 
-size_t pi0hip_vision_attention_workspace_bytes(int views, int heads) {
-  if (views <= 0 || heads <= 0) return 0;
-  return round256_((size_t)views * heads * VA_HDP * VA_TOK * sizeof(__bf16));
-}
+size_t pi0hip_vision_attention_workspace_bytes(int, int) { return 0; }
 
 int pi0hip_vision_attention(const void* qkv, int ldqkv, void* out, int ldo, int views, int tokens,
-                            int heads, int head_dim, float scale, void* ws, size_t ws_bytes,
-                            hipStream_t s) {
+                            int heads, int head_dim, float scale, void*, size_t, hipStream_t s) {
   if (!qkv || !out || views <= 0 || heads <= 0) return PI0HIP_ERR_ARG;
   const int dim = heads * head_dim;
   if (tokens != VA_TOK || head_dim != VA_HD || ldqkv < 3 * dim || ldo < dim ||
-      misaligned(qkv, ldqkv) || (ldo & 3) || (reinterpret_cast<uintptr_t>(out) & 7))
+      misaligned(qkv, ldqkv) || (ldo & 3) || (reinterpret_cast<uintptr_t>(out) & 7) ||
+      (long long)VA_TOK * ldqkv * (long long)sizeof(__bf16) > INT_MAX)
     return PI0HIP_ERR_SHAPE;
-  if (!ws || ws_bytes < pi0hip_vision_attention_workspace_bytes(views, heads))
-    return PI0HIP_ERR_WORKSPACE;
-  hipLaunchKernelGGL(vision_vt_kernel, dim3(VA_TOK / 64, heads, views), dim3(256), 0, s,
-                     (const __bf16*)qkv, ldqkv, (__bf16*)ws, heads, dim);
-  if (hipError_t e = hipGetLastError()) return (int)e;
   VisAttnArgs a = {};
   a.qkv = (const __bf16*)qkv; a.ldqkv = ldqkv;
-  a.vt = (const __bf16*)ws;
   a.out = (__bf16*)out; a.ldo = ldo;
-  a.heads = heads; a.dim = dim;
+  a.dim = dim;
   a.scale_log2 = 1.4426950408889634f * scale;
-  // two 32-query tiles of one (view, head) per workgroup: their identical K / V^T fragment
-  // loads meet in one CU's L1 (3 views: 14.5 -> 13.8 us with the V^T pass, 12 views:
-  // 37.9 -> 35.8; four tiles: 17.9 / 35.3)
-  hipLaunchKernelGGL(vision_attn_kernel<2>, dim3(VA_TOK / 64, heads, views), dim3(128), 0, s, a);
+  hipLaunchKernelGGL(vision_attn_kernel, dim3(VA_TOK / (32 * VA_QT), heads, views),
+                     dim3(64 * VA_QT * VA_KS), 0, s, a);
   return (int)hipGetLastError();
 }
 

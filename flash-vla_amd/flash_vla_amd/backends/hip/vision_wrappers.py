@@ -9,8 +9,6 @@ the valid output columns are stored.
 """
 from __future__ import annotations
 
-import torch
-
 from . import _abi
 from .wrappers import _check, _ptr, _stream, packed_weight_ptr, scratch
 
@@ -104,10 +102,8 @@ def vision_attention(QKV):
     views = QKV.shape[0] if QKV.dim() == 3 else QKV.shape[0] // TOKENS
     q2 = _rows(QKV, 3 * DIM)
     out = scratch("vision_attn_out", (views, TOKENS, DIM), QKV.dtype, QKV.device)
-    nbytes = _abi.lib().pi0hip_vision_attention_workspace_bytes(views, HEADS)
-    ws = scratch("vision_attn_ws", (nbytes,), torch.uint8, QKV.device)
     _abi.call("pi0hip_vision_attention", _ptr(q2), q2.stride(0), _ptr(out), DIM, views, TOKENS,
-              HEADS, HEAD_DIM, HEAD_DIM ** -0.5, ws.data_ptr(), nbytes, _stream())
+              HEADS, HEAD_DIM, HEAD_DIM ** -0.5, None, 0, _stream())
     return out
 
 

@@ -350,7 +350,7 @@ int pi0hip_tile_linear_bias_gelu(const void* x, int ldx, const void* w_packed, c
  * The patchify of vision_patch_embed (wrappers.py:257-269). */
 int pi0hip_im2col_patches(const void* images, int views, void* out, int ldo, hipStream_t s);
 
-/* Workspace of pi0hip_vision_attention: per-head transposed V. */
+/* Workspace of pi0hip_vision_attention: none is needed (0), `ws` may be null. */
 size_t pi0hip_vision_attention_workspace_bytes(int views, int heads);
 
 /* Per view and head: out = softmax(scale * q k^T) v over the view's 256 tokens, q / k / v

@@ -1,0 +1,35 @@
+"""Vision attention from LDS: views, magnitudes and masked-like keys against 64 bits.
+
+P is rounded to bf16 (2^-9 relative each) and so is the output: with 256 keys the P roundings
+average out below one output rounding, so 2^-7 of a row's largest value covers both."""
+import pytest
+import torch
+
+from flash_vla_amd.arena import ScratchPool
+from flash_vla_amd.backends.hip import vision_wrappers as VW
+from flash_vla_amd.backends.hip import wrappers as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _ref(qkv):
+    n = qkv.shape[0]
+    q, k, v = qkv.double().reshape(n, 256, 3, 16, 72).permute(2, 0, 3, 1, 4)
+    p = torch.softmax(q @ k.transpose(-1, -2) / 72 ** 0.5, -1)
+    return (p @ v).transpose(1, 2).reshape(n, 256, 1152)
+
+
+@pytest.mark.parametrize("views", [1, 4, 13])
+@pytest.mark.parametrize("scale", [0.0, 1.0, 6.0])       # flat, ordinary, nearly one-hot
+def test_against_64_bits(views, scale):
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    g = torch.Generator(device="cuda").manual_seed(views)
+    qkv = torch.randn(views, 256, 3456, generator=g, device="cuda")
+    qkv[..., :2304] *= scale
+    qkv[:, 100:140, 1152:2304] -= 4 * scale              # a run of keys that most queries skip
+    qkv = qkv.bfloat16()
+    with W.use_pool(ScratchPool()):
+        out = VW.vision_attention(qkv)
+    ref = _ref(qkv)
+    assert torch.all((out.double() - ref).abs() <= 2.0 ** -7 * ref.abs().amax(-1, keepdim=True))
