@@ -168,3 +168,24 @@ def test_batched_gate_rows(M):
         W.decoder_norm_gated_ffn(x[r:r + n], g, u, part, None)
         assert torch.equal(out[r:r + n], part)
     assert torch.all(out[M:] == 7.0), "stored past row M"
+
+
+@pytest.mark.parametrize("B,L", [(3, 769), (8, 256), (5, 415), (2, 815)])
+@pytest.mark.parametrize("scale", [1.0, 6.0])           # ordinary, nearly one-hot
+def test_encoder_attention_many_rows(B, L, scale):
+    """The 128-row workgroups (from 128 of them on; the last case stays below) against 64 bits:
+    P's and the output's bf16 roundings, 2^-9 each, and the smaller form's bf16 logits."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    from flash_vla_amd.arena import ScratchPool
+    from flash_vla_amd.backends.hip import encoder_wrappers as EW
+    q, k, v = rnd((B * L * 8, 256), 28, scale), rnd((B, L, 256), 29), rnd((B, L, 256), 30)
+    with W.use_pool(ScratchPool()):
+        out = EW.encoder_attention(q, k, v, 1 / 16).reshape(B, L * 8, 256).double()
+    wide = B * ((L * 8 + 127) // 128) >= 128
+    p = torch.softmax(q.double().reshape(B, L * 8, 256) @ k.double().transpose(1, 2) / 16, -1)
+    ref = p @ v.double()
+    err = ((out - ref).norm() / ref.norm()).item()
+    # bf16 logits: 2^-9 of a logit of about 4 scale, so 4 scale 2^-9 on P
+    assert err <= (4e-3 if wide else 4e-3 + scale * 2.0 ** -7), err
+    assert torch.isfinite(out).all()
