@@ -78,6 +78,27 @@ def check_kblock_waits(asm: str) -> list[str]:
     return bad
 
 
+# kernels whose every copy lies inside its resource, whatever the call's sizes
+_COPIES_IN_RANGE = ("enc_attn_wide_kernel",)      # clamped blocks of the packed K and V^T
+
+
+def unchecked_copies(asm: str) -> list[str]:
+    """Names of kernels with a buffer load into LDS whose scalar offset is not zero.
+
+    Rows past M, and the columns past a row's end that a padded K asks for, rely on the range
+    check of the activation's buffer resource. The check is documented for the lane and the
+    immediate offset only, so nothing may sit in the scalar one."""
+    bad = []
+    for m in re.finditer(r"^(_ZN3pi0\w+):", asm, re.M):
+        body = asm[m.end():asm.index("s_endpgm", m.end())]
+        copies = [ln.split(";")[0].rstrip() for ln in body.split("\n")
+                  if re.match(r"\s*buffer_load\w*\s.*\blds\b", ln)]
+        soffs = {ln.split(",")[-1].split()[0] for ln in copies}
+        if soffs - {"0"} and not any(k in m.group(1) for k in _COPIES_IN_RANGE):
+            bad.append(m.group(1))
+    return bad
+
+
 def scratch_kernels(asm: str) -> list[str]:
     """Kernels whose private (scratch) segment is not empty: a spill, or a kernel argument
     indexed at run time and so copied to the stack -- both silent slowdowns."""
@@ -91,8 +112,8 @@ def scratch_kernels(asm: str) -> list[str]:
 
 def check_device_code(src: str) -> None:
     """Compile `src` to device assembly and fail if any packed fp32 VALU op was
-    generated, if any kernel uses scratch memory, or (pi0_gemm.hip) if a skinny GEMM's
-    k-block waits are unsafe."""
+    generated, if any kernel uses scratch memory, if a copy into LDS could leave its
+    resource's range check, or (pi0_gemm.hip) if a skinny GEMM's k-block waits are unsafe."""
     cmd = [HIPCC, *FLAGS, "--cuda-device-only", "-S", src, "-o", "-"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
@@ -102,6 +123,9 @@ def check_device_code(src: str) -> None:
     scratch = scratch_kernels(res.stdout)
     if scratch:
         raise RuntimeError(f"{src}: kernels with a scratch segment: {scratch}")
+    loose = unchecked_copies(res.stdout)
+    if loose:
+        raise RuntimeError(f"{src}: LDS copies outside the range check in {loose}")
     if os.path.basename(src) == "pi0_gemm.hip":
         bad = check_kblock_waits(res.stdout)
         if bad:

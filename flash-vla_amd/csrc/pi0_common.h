@@ -98,7 +98,16 @@ __device__ __forceinline__ void buf_load16_lds(__amdgpu_buffer_rsrc_t r, void* l
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds_base,
                                            16, off, 0, 0, 0);
 }
-// The same with a wave-uniform byte offset `soff` (an SGPR) added to the lane offset.
+// The same with a wave-uniform byte offset `soff` added to the lane offset. The sum is the lane
+// offset of the instruction: its own scalar offset is not a documented part of the range check,
+// and copies rely on that check for the rows past M and the padded end of K. (readfirstlane
+// keeps the compiler from folding soff's loop-invariant parts into further lane registers:
+// 384-row blocks spilled with them.)
+__device__ __forceinline__ void buf_load16_lds_u(__amdgpu_buffer_rsrc_t r, void* lds_base, int off,
+                                                 int soff) {
+  buf_load16_lds(r, lds_base, off + __builtin_amdgcn_readfirstlane(soff));
+}
+// ... and with `soff` as the scalar offset, for copies that lie inside the resource.
 __device__ __forceinline__ void buf_load16_lds_s(__amdgpu_buffer_rsrc_t r, void* lds_base, int off,
                                                  int soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds_base,

@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(TileArgs a) {
     const int abase = st * 64 * (int)sizeof(__bf16);
 #pragma unroll
     for (int i = 0; i < LA; ++i)
-      buf_load16_lds_s(ar, &lds[(slot * TA + i * 4 + wave) * 64], aoff, abase + i * arow_step);
+      buf_load16_lds_u(ar, &lds[(slot * TA + i * 4 + wave) * 64], aoff, abase + i * arow_step);
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
@@ -447,11 +447,11 @@ __global__ __launch_bounds__(64 * WMC * WNC, 1) void block_gemm_kernel(TileArgs 
     bf16x8* const da = &lds[A0 + slot * SA + q * 64];
     bf16x8* const db = &lds[slot * SB + qb * 64];
     if (i * NW + NW <= TA)
-      buf_load16_lds_s(ar, da, avoff, soff);
+      buf_load16_lds_u(ar, da, avoff, soff);
     else if (i * NW >= TA)
-      buf_load16_lds_s(up ? ur : gr, db, bvoff, soff);
+      buf_load16_lds_u(up ? ur : gr, db, bvoff, soff);
     else                                                 // both kinds: B's first tiles
-      buf_load16_lds_s(isa ? ar : gr, isa ? da : db, isa ? avoff : bvoff, soff);
+      buf_load16_lds_u(isa ? ar : gr, isa ? da : db, isa ? avoff : bvoff, soff);
   };
 
   f32x16 acc[FM][FN];
@@ -632,7 +632,7 @@ __global__ __launch_bounds__(512, 1) void rows32_res_kernel(TileArgs a, int nrb,
   auto copy = [&](int c) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      buf_load16_lds_s(xr, xs + (c % SL) * 256 + i * 64,
+      buf_load16_lds_u(xr, xs + (c % SL) * 256 + i * 64,
                        xoff + ((lane & 7) ^ ((i & 1) * 4 + (lane >> 4))) * 16,
                        c * 128 + i * 8 * a.lda * (int)sizeof(__bf16));
   };

@@ -529,7 +529,7 @@ __global__ __launch_bounds__(512, 1) void gate_stream_kernel(GemmArgs a) {
   auto copy = [&](int j, int c) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      buf_load16_lds_s(xr, xs + c * 256 + i * 64,
+      buf_load16_lds_u(xr, xs + c * 256 + i * 64,
                        xoff + ((lane & 7) ^ ((i & 1) * 4 + (lane >> 4))) * 16,
                        c * 128 + ((2 * j + rh) * 32 + i * 8) * a.ldx * (int)sizeof(__bf16));
     __builtin_amdgcn_sched_barrier(0);

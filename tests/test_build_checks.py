@@ -21,13 +21,22 @@ pytestmark = pytest.mark.skipif(not os.path.exists(build_lib.HIPCC) and not shut
                                 reason="needs hipcc")
 
 
-@pytest.fixture(scope="module")
-def gemm_asm():
-    src = os.path.join(build_lib.CSRC, "pi0_gemm.hip")
+def _asm(name):
+    src = os.path.join(build_lib.CSRC, name)
     res = subprocess.run([build_lib.HIPCC, *build_lib.FLAGS, "--cuda-device-only", "-S", src,
                           "-o", "-"], capture_output=True, text=True)
     assert res.returncode == 0, res.stderr
     return res.stdout
+
+
+@pytest.fixture(scope="module")
+def gemm_asm():
+    return _asm("pi0_gemm.hip")
+
+
+@pytest.fixture(scope="module")
+def encoder_asm():
+    return _asm("pi0_encoder.hip")
 
 
 def test_kblock_waits_hold(gemm_asm):
@@ -48,6 +57,17 @@ def test_kblock_waits_reject_a_loose_wait(gemm_asm, name):
     first = body.index("s_waitcnt vmcnt(", body.index(" lds\n"))   # first k-block wait
     loose = body[:first] + "s_waitcnt vmcnt(60)" + body[body.index(")", first) + 1:]
     assert build_lib.check_kblock_waits(gemm_asm.replace(body, loose)) == [name]
+
+
+def test_activation_copies_stay_inside_the_range_check(gemm_asm, encoder_asm):
+    """Rows past M and the columns past a padded K's end are zeros because the copy's whole
+    offset is the lane's (see build_lib.unchecked_copies)."""
+    assert "block_gemm_kernel" in encoder_asm and "rows32_res_kernel" in encoder_asm
+    assert build_lib.unchecked_copies(encoder_asm) == []
+    assert build_lib.unchecked_copies(gemm_asm) == []
+    fake = "_ZN3pi07k_looseEv:\n\tbuffer_load_dwordx4 v1, s[0:3], s9 offen lds\n\ts_endpgm\n"
+    assert build_lib.unchecked_copies(fake) == ["_ZN3pi07k_looseEv"]
+    assert build_lib.unchecked_copies(fake.replace("s9", "0")) == []
 
 
 def test_no_packed_fp32(gemm_asm):

@@ -98,3 +98,18 @@ def test_bias_gelu_and_bias_ragged(M):
     torch.cuda.synchronize()
     _check(out2[:M], (x.float() @ w2.float() + b2.float()).bfloat16(), f"bias M={M}")
     assert torch.all(out2[M:] == 7.0), "stored past row M"
+
+
+@pytest.mark.parametrize("M", [100, 1025, 2100])       # 32-, 64- and 128-row tiles
+def test_padded_k_ends_at_the_last_row(M):
+    """The FFN-down's 48 padding columns of the last row lie past the activation: they must
+    read as zeros whatever memory holds there (0 x NaN would reach that row's outputs)."""
+    K, N, K_pad = 4304, 1152, 4352
+    x = rnd((M + 8, K), 13)
+    x[M:] = float("nan")
+    w, b, res = rnd((K, N), 14, 0.02), rnd(N, 15, 0.5), rnd((M, N), 16)
+    out = torch.empty_like(res)
+    _abi.call("pi0hip_tile_linear_bias_res", x.data_ptr(), K, W.packed_weight_ptr(w, 32, (K_pad, N)),
+              b.data_ptr(), res.data_ptr(), N, 0, out.data_ptr(), N, M, N, K, N, K_pad, W._stream())
+    torch.cuda.synchronize()
+    _check(out, (x[:M].float() @ w.float() + b.float() + res.float()).bfloat16(), f"ffn down M={M}")
