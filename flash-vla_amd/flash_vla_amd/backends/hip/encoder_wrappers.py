@@ -21,12 +21,13 @@ LN_EPS = 1e-5
 
 def _down_splitk(M: int, K: int) -> int:
     """K splits of the ffn-down (K = 16384, N = 2048), partials summed in split order by a second
-    launch: as many as fill the 256 CUs for one round with the tile that the library then picks.
-    us with 4 splits (1 from 2048 rows) -> now: 269 rows 48.7 -> 36.6 (8), 512 54.8 -> 51.1 (8),
-    816 95.8 -> 70.4 (8), 1024 100.8 -> 76.4 (8), 1280 110.6 -> 97.7 (4), 1632 153 -> 110 (4);
-    768 rows stay on 4 (63.1 against 65.0 with 8)."""
+    launch. Four fill the 256 CUs from 512 rows on, and a request of that many tokens keeps its
+    sums' order, so its bits, in any batch up to 3072 rows. Between 256 and 512 rows four leave
+    half of the chip idle. us with 8 / 4 splits: 269 rows 36.0 / 48.8, 400 42.2 / 54.2, 512
+    51.4 / 54.1, 560 59.1 / 54.8, 816 71.6 / 66.8, 896 74.3 / 79.8, 1024 81.3 / 82.2, 1632
+    137 / 116; 256 rows 46.9 / 45.2. Unsplit from 3073 rows (3264: 215)."""
     if K % 1024 == 0:
-        if 256 < M <= 640 or 768 < M <= 1024:
+        if 256 < M < 512:
             return 8
         return 4 if M <= 3072 else 1
     return 4 if (K // 64) % 4 == 0 and M < 2048 else 1

@@ -1,10 +1,11 @@
 """Batch-4 / prompt-token profile (not in the reference, which is
 batch-1 with precomputed language embeddings).
 
-The batched kernels must give every request exactly what a batch-1 run of that request
-gives: each row's arithmetic does not depend on how rows are grouped into blocks, so the
-checks are bitwise (Q / K / V scatter, RoPE positions, per-request caches, the attention's
-state-row mask and its "states first" output order). The batched forward is also checked
+Each row's arithmetic does not depend on how rows are grouped into blocks, so the checks of
+Q / K / V scatter, RoPE positions, per-request caches, the attention's state-row mask and its
+"states first" output order are bitwise against batch-1 runs, and so are whole encoder layers
+where the attention and the down projection's split are the single request's (two requests of
+768 or 816 tokens; larger batches take the wide attention, compared at rounding). The batched forward is also checked
 against the CPU oracle run request by request (relative criterion as for the full forward).
 """
 import pytest
@@ -96,6 +97,33 @@ def test_encoder_qkv_and_attention_batched_equal_per_request():
         a1 = EW.encoder_attention(qb, k1, v1, 256 ** -0.5)
         assert torch.equal(a1, att[b * Lp:(b + 1) * Lp])
     assert not ck[:, 1, Lp:].any(), "wrote decoder rows"
+
+
+@pytest.mark.parametrize("tokens,B", [(816, 2), (768, 2)])
+def test_encoder_layers_batched_equal_per_request(tokens, B):
+    """Whole encoder layers: the K / V of the last of three layers follow from two layers'
+    attention, o-proj, gated FFN and down projection."""
+    from flash_vla_amd import op_table, pipeline
+    from flash_vla_amd.buffers import allocate_encoder_buffers
+    n, ops = 3, op_table(True)
+    shapes = {"encoder_attn_qkv_w": (2048, 2560), "encoder_attn_o_w": (2048, 2048),
+              "encoder_ffn_gate_w": (2048, 16384), "encoder_ffn_up_w": (2048, 16384),
+              "encoder_ffn_down_w": (16384, 2048)}
+    g = torch.Generator(device=DEV).manual_seed(115)
+    w = {k: (torch.randn(n, *s, generator=g, device=DEV) * 0.02).to(torch.bfloat16)
+         for k, s in shapes.items()}
+    x = rnd((B, tokens, 2048), 116)
+
+    def run(xs):
+        b = allocate_encoder_buffers(tokens, DEV, layers=n, batch=xs.shape[0])
+        b["encoder_x"].copy_(xs.reshape(-1, 2048))
+        pipeline.transformer_encoder(ops, w, b, tokens, project=False)
+        return b["encoder_K"].view(-1, n, tokens, 256), b["encoder_V"].view(-1, n, tokens, 256)
+
+    k, v = run(x)
+    for b in range(B):
+        k1, v1 = run(x[b:b + 1])
+        assert torch.equal(k[b], k1[0]) and torch.equal(v[b], v1[0]), f"request {b}"
 
 
 def test_embed_prompt():

@@ -10,6 +10,7 @@ from flash_vla_amd import op_table
 from flash_vla_amd.arena import ScratchPool
 from flash_vla_amd.backends import BACKENDS, register_backend
 from flash_vla_amd.backends.hip import _abi, wrappers
+from flash_vla_amd.backends.hip.encoder_wrappers import _down_splitk
 from flash_vla_amd.spec import decoder_weight_shapes, weight_shapes
 
 ROOT = Path(__file__).resolve().parents[1]
@@ -121,6 +122,13 @@ def test_splitk_choice_fills_the_chip():
     for M, N, K in [(51, 1024, 2048), (50, 32, 1024), (51, 2560, 1024), (204, 1024, 4096)]:
         s = wrappers._splitk(M, N, K)
         assert (K // 32) % (4 * s) == 0
+
+
+@pytest.mark.parametrize("tokens,batch", [(816, 2), (816, 3), (768, 4), (1023, 3), (512, 6), (256, 12)])
+def test_down_split_of_a_batch_is_the_single_request_s(tokens, batch):
+    """The split decides the order of the sums: with another one a request's rows in a batch
+    are not bit for bit those of the request alone."""
+    assert _down_splitk(tokens * batch, 16384) == _down_splitk(tokens, 16384)
 
 
 def test_schema_shapes():
