@@ -1441,7 +1441,6 @@ static int launch_block(TileArgs a, hipStream_t s) {
 
 static int launch_rows32(const TileArgs& a, hipStream_t s) {
   const int nrb = (a.M + 31) / 32, ntiles = a.N / 32, xcd_map = ntiles % 8 == 0;
-  if (a.N % 32) return PI0HIP_ERR_SHAPE;
   switch (a.K) {
     case 2048: hipLaunchKernelGGL(rows32_res_kernel<16>, dim3(nrb * ntiles), dim3(512), 0, s, a, nrb, xcd_map); break;
     case 4096: hipLaunchKernelGGL(rows32_res_kernel<32>, dim3(nrb * ntiles), dim3(512), 0, s, a, nrb, xcd_map); break;
@@ -1582,7 +1581,7 @@ int pi0hip_tile_linear_residual(const void* x, int ldx, const void* w_packed, vo
     // The batched decoder's o-proj and down (N = 1024, K 2048 / 4096): 32 x 32 workgroups over
     // the whole K, 204 rows 8.5 -> 4.9 and 11.2 -> 8.1 against 4 splits and their sum, 408
     // rows 15.5 -> 8.1 and 20.8 -> 14.8.
-    const bool rows32 = (K == 2048 || K == 4096) && N % 32 == 0;
+    const bool rows32 = (K == 2048 || K == 4096) && N % 128 == 0;   // whole tiles, as the others
     switch (least({tile_us(M, N, 64, 128, 13.3f), block_us(M, N, K, 128, 128, 20.5f),
                    block_us(M, N, K, 128, 256, 28.5f), block_us(M, N, K, 192, 256, 42.f),
                    block_us(M, N, K, 256, 256, 56.f), tile_us(M, N, 32, 128, 8.3f),

@@ -60,6 +60,9 @@ def test_rejected_arguments_do_not_launch():
     assert lib.pi0hip_linear_residual(1, 2048, 1, 1, 1024, 51, 1024, 2048, 4, None, 0,
                                       None) == -3
     assert lib.pi0hip_norm_gated_ffn(1, 1024, 1, 1, 1, 4096, 51, 4096, 1000, None) == -2
+    # a residual projection is whole 128-column tiles, at few rows too
+    for m, n, k in [(64, 96, 2048), (64, 32, 4096), (512, 96, 2048), (64, 96, 1024)]:
+        assert lib.pi0hip_tile_linear_residual(16, k, 16, 16, n, m, n, k, 1, None, 0, None) == -2
     with pytest.raises(_abi.HipLibraryError):
         _abi.check(-2, "x")
 
