@@ -1454,15 +1454,18 @@ static int launch_rows32(const TileArgs& a, hipStream_t s) {
 // choice is the least rounds x (measured length of a full round). The lengths are single
 // launches with cold weights in a graph; what matters is their ratio, which K does not change
 // much. Kernels that share a CU (per_cu 2) refill it as they end, without rounds.
-static float tile_us(int M, int N, int bm, int bn, float round_us, int splitk = 1, int per_cu = 1) {
-  const float w = (float)((M + bm - 1) / bm) * (float)((N + bn - 1) / bn) * (float)splitk;
+// A tile whose rows lie further apart than 32-bit buffer offsets reach is no choice.
+static float tile_us(const TileArgs& a, int bm, int bn, float round_us, int per_cu = 1) {
+  if ((long long)bm * a.lda * (long long)sizeof(__bf16) > INT_MAX) return INFINITY;
+  const float w = (float)((a.M + bm - 1) / bm) * (float)((a.N + bn - 1) / bn) * (float)a.splitk;
   const float r = w / (float)(per_cu * device_cus());
   return round_us * (per_cu > 1 ? fmaxf(r, 0.8f) : ceilf(r));
 }
-// ... of a block_gemm_kernel tile, which needs whole column tiles and 128-deep K
-static float block_us(int M, int N, int K, int bm, int bn, float round_us, int splitk = 1) {
-  if (N % bn || K % (128 * splitk)) return INFINITY;
-  return tile_us(M, N, bm, bn, round_us, splitk);
+// ... of a block_gemm_kernel tile, which needs whole column tiles and 128-deep K (launch_block)
+static float block_us(const TileArgs& a, int bm, int bn, float round_us) {
+  if (a.N % bn || a.K % (128 * a.splitk) || (long long)a.K * 256 * (long long)sizeof(__bf16) > INT_MAX)
+    return INFINITY;
+  return tile_us(a, bm, bn, round_us);
 }
 static int least(std::initializer_list<float> us) {
   return (int)(std::min_element(us.begin(), us.end()) - us.begin());
@@ -1489,10 +1492,10 @@ static bool misaligned(const void* p, int ld) {
 template <int EPI>
 static int linear_launch(const TileArgs& a, hipStream_t s) {
   const bool d3 = a.K % 192 == 0;
-  switch (least({tile_us(a.M, a.N, 64, 128, 8.5f), tile_us(a.M, a.N, 32, 128, 6.7f),
-                 d3 ? tile_us(a.M, a.N, 96, 128, 10.4f) : INFINITY,
-                 d3 ? tile_us(a.M, a.N, 96, 128, 21.2f, 1, 2) : INFINITY,
-                 block_us(a.M, a.N, a.K, 128, 128, 12.3f), block_us(a.M, a.N, a.K, 256, 128, 22.f)})) {
+  switch (least({tile_us(a, 64, 128, 8.5f), tile_us(a, 32, 128, 6.7f),
+                 d3 ? tile_us(a, 96, 128, 10.4f) : INFINITY,
+                 d3 ? tile_us(a, 96, 128, 21.2f, 2) : INFINITY,
+                 block_us(a, 128, 128, 12.3f), block_us(a, 256, 128, 22.f)})) {
     case 1: return launch_tile_d4<32, 32, EPI, false>(a, s);
     case 2: case 3: return launch_tile<96, 32, 3, EPI, false, 2>(a, s);
     case 4: return launch_block<4, 2, 1, 2, EPI>(a, s);
@@ -1505,11 +1508,11 @@ static int linear_launch(const TileArgs& a, hipStream_t s) {
 static int partial_launch(const TileArgs& a, hipStream_t s) {
   // small M (the batched decoder, 204 rows): 32-row tiles, two workgroups per CU
   if (a.M <= 256) return launch_tile_auto<32, 32, 4, TE_PARTIAL, false, 2>(a, s);
-  switch (least({tile_us(a.M, a.N, 192, 128, 57.f, a.splitk),
-                 block_us(a.M, a.N, a.K, 128, 256, 62.f, a.splitk),
-                 block_us(a.M, a.N, a.K, 192, 256, 92.f, a.splitk),
-                 block_us(a.M, a.N, a.K, 256, 256, 112.f, a.splitk),
-                 block_us(a.M, a.N, a.K, 384, 256, 155.f, a.splitk)})) {
+  switch (least({tile_us(a, 192, 128, 57.f),
+                 block_us(a, 128, 256, 62.f),
+                 block_us(a, 192, 256, 92.f),
+                 block_us(a, 256, 256, 112.f),
+                 block_us(a, 384, 256, 155.f)})) {
     case 1: return launch_block<2, 4, 2, 2, TE_PARTIAL>(a, s);
     case 2: return launch_block<2, 4, 3, 2, TE_PARTIAL>(a, s);
     case 3: return launch_block<4, 2, 2, 4, TE_PARTIAL>(a, s);
@@ -1574,7 +1577,7 @@ int pi0hip_tile_linear_residual(const void* x, int ldx, const void* w_packed, vo
     // while that grid fits one round (3264 rows 217 us against 276 for the same block of
     // block_gemm_kernel); past it 256 x 256 blocks, 6528 rows 475 -> 393.
     if (K >= 8192 && M >= 2048 && N % 256 == 0) {
-      if (block_us(M, N, K, 256, 256, 393.f) < tile_us(M, N, 128, 256, 225.f))
+      if (block_us(a, 256, 256, 393.f) < tile_us(a, 128, 256, 225.f))
         return launch_block<4, 2, 2, 4, TE_RES>(a, s);
       return launch_tile_d4<128, 64, TE_RES, false>(a, s);
     }
@@ -1582,10 +1585,10 @@ int pi0hip_tile_linear_residual(const void* x, int ldx, const void* w_packed, vo
     // the whole K, 204 rows 8.5 -> 4.9 and 11.2 -> 8.1 against 4 splits and their sum, 408
     // rows 15.5 -> 8.1 and 20.8 -> 14.8.
     const bool rows32 = (K == 2048 || K == 4096) && N % 128 == 0;   // whole tiles, as the others
-    switch (least({tile_us(M, N, 64, 128, 13.3f), block_us(M, N, K, 128, 128, 20.5f),
-                   block_us(M, N, K, 128, 256, 28.5f), block_us(M, N, K, 192, 256, 42.f),
-                   block_us(M, N, K, 256, 256, 56.f), tile_us(M, N, 32, 128, 8.3f),
-                   rows32 ? tile_us(M, N, 32, 32, 5.2f) : INFINITY})) {
+    switch (least({tile_us(a, 64, 128, 13.3f), block_us(a, 128, 128, 20.5f),
+                   block_us(a, 128, 256, 28.5f), block_us(a, 192, 256, 42.f),
+                   block_us(a, 256, 256, 56.f), tile_us(a, 32, 128, 8.3f),
+                   rows32 ? tile_us(a, 32, 32, 5.2f) : INFINITY})) {
       case 1: return launch_block<4, 2, 1, 2, TE_RES>(a, s);
       case 2: return launch_block<2, 4, 2, 2, TE_RES>(a, s);
       case 3: return launch_block<2, 4, 3, 2, TE_RES>(a, s);
@@ -1618,9 +1621,9 @@ int pi0hip_tile_gated_ffn(const void* x, int ldx, const void* gate_packed, const
   // above, blocks of 192, 256 or 384 rows x 128 outputs. us before -> after with the encoder's
   // N = 16384, K = 2048: 269 rows 62.6 -> 48.1, 400 67 -> 59, 768 93 -> 89, 816 142 -> 108,
   // 1024 148 -> 119, 3264 396 -> 380, 6528 771 -> 730.
-  if (M > 256 && N % 128 == 0 && K % 128 == 0)
-    switch (least({block_us(M, N, K, 192, 128, 50.f), block_us(M, N, K, 256, 128, 58.f),
-                   block_us(M, N, K, 384, 128, 86.f)})) {
+  if (M > 256 && std::isfinite(block_us(a, 192, 128, 50.f)))
+    switch (least({block_us(a, 192, 128, 50.f), block_us(a, 256, 128, 58.f),
+                   block_us(a, 384, 128, 86.f)})) {
       case 0: return launch_block<2, 4, 3, 2, TE_GATE, true>(a, s);
       case 1: return launch_block<4, 2, 2, 4, TE_GATE, true>(a, s);
       default: return launch_block<4, 2, 3, 4, TE_GATE, true>(a, s);
@@ -1662,9 +1665,9 @@ int pi0hip_tile_qkv_rope_batched(const void* x, int ldx, const void* w_packed, c
   a.rows_per_batch = rows_per_batch; a.kv_bstride = kv_bstride;
   // us before -> after at N = 2560, K = 2048: 816 rows 24.3 -> 17.3 (260 workgroups of 64 x 128
   // are two rounds), 1632 29.7 -> 24.8, 3264 53.4 -> 36.9, 6528 94 -> 67
-  switch (least({tile_us(M, a.N, 64, 128, 13.f), block_us(M, a.N, K, 128, 128, 18.f),
-                 block_us(M, a.N, K, 128, 256, 27.f), block_us(M, a.N, K, 192, 256, 38.f),
-                 block_us(M, a.N, K, 256, 256, 48.f)})) {
+  switch (least({tile_us(a, 64, 128, 13.f), block_us(a, 128, 128, 18.f),
+                 block_us(a, 128, 256, 27.f), block_us(a, 192, 256, 38.f),
+                 block_us(a, 256, 256, 48.f)})) {
     case 1: return launch_block<4, 2, 1, 2, TE_QKV_ROPE>(a, s);
     case 2: return launch_block<2, 4, 2, 2, TE_QKV_ROPE>(a, s);
     case 3: return launch_block<2, 4, 3, 2, TE_QKV_ROPE>(a, s);
@@ -1749,8 +1752,8 @@ int pi0hip_tile_linear_bias_res(const void* x, int ldx, const void* w_packed, co
   // M = 768, 17.3 against 19.2 at M = 3072. Rows per tile by the rounds they make (relative
   // round lengths; o-proj at 1536 rows 11.5 -> 9.2 us, FFN-down 36.0 -> 34.2).
   const bool d3 = (K_pad / 64) % 3 == 0 && (K_pad / 64) % 4 != 0;
-  switch (least({tile_us(M, N_pad, 32, 128, 1.f), tile_us(M, N_pad, 64, 128, 1.42f),
-                 tile_us(M, N_pad, 128, 128, 2.05f)})) {
+  switch (least({tile_us(a, 32, 128, 1.f), tile_us(a, 64, 128, 1.42f),
+                 tile_us(a, 128, 128, 2.05f)})) {
     case 0: return d3 ? launch_tile<32, 32, 3, TE_BIAS_RES, false, 1>(a, s)
                       : launch_tile_auto<32, 32, 8, TE_BIAS_RES, false>(a, s);
     case 1: return d3 ? launch_tile<64, 32, 3, TE_BIAS_RES, false, 1>(a, s)
@@ -1774,9 +1777,9 @@ int pi0hip_tile_linear_bias_gelu(const void* x, int ldx, const void* w_packed, c
   // (768 rows 16.3 us), then blocks by the rounds they make. us before -> after: 2048 rows
   // 39.1 -> 32.2, 3072 50.3 -> 40.3, 4096 63.8 -> 55.7, 6144 86.6 -> 78.0.
   const bool d3 = N_pad % 128 == 0 && K_pad % 192 == 0;
-  switch (least({d3 ? tile_us(M, N_pad, 64, 128, 17.f, 1, 2) : INFINITY,
-                 block_us(M, N_pad, K_pad, 128, 256, 26.5f), block_us(M, N_pad, K_pad, 192, 256, 33.f),
-                 block_us(M, N_pad, K_pad, 256, 256, 40.f), block_us(M, N_pad, K_pad, 384, 256, 56.f),
+  switch (least({d3 ? tile_us(a, 64, 128, 17.f, 2) : INFINITY,
+                 block_us(a, 128, 256, 26.5f), block_us(a, 192, 256, 33.f),
+                 block_us(a, 256, 256, 40.f), block_us(a, 384, 256, 56.f),
                  1e30f})) {
     case 0: return launch_tile<64, 32, 3, TE_BIAS_GELU, false, 2>(a, s);
     case 1: return launch_block<2, 4, 2, 2, TE_BIAS_GELU>(a, s);

@@ -1079,7 +1079,9 @@ int pi0hip_norm_gated_ffn(const void* x, int ldx, const void* gate_p, const void
   if (!x || !gate_p || !up_p || !out) return PI0HIP_ERR_ARG;
   GemmArgs a = base_args(x, ldx, gate_p, out, ldo, M, N, K, 1);
   a.w1 = (const __bf16*)up_p;
-  if (M > 64 && M <= 256 && K == 1024 && N > 0 && N % 16 == 0) {
+  // (one buffer resource holds all rows: 32-bit offsets have to reach the last)
+  if (M > 64 && M <= 256 && K == 1024 && N > 0 && N % 16 == 0 &&
+      (long long)M * ldx * (long long)sizeof(__bf16) <= INT_MAX) {
     if (bad_alignment(a)) return PI0HIP_ERR_SHAPE;
     const dim3 grid(N / 16), block(512);
     if (M <= 128) hipLaunchKernelGGL(gate_stream_kernel<2>, grid, block, 0, s, a);

@@ -47,6 +47,32 @@ def test_gated_ffn_blocks(M):
         W._stream()))
 
 
+def _wide(x, pitch):
+    """x's rows `pitch` elements apart (gigabytes, of which only the rows are touched)."""
+    w = torch.empty(x.shape[0] * pitch, dtype=x.dtype, device=DEV).view(-1, pitch)[:, :x.shape[1]]
+    w.copy_(x)
+    return w
+
+
+def test_wide_row_pitches():
+    """A pitch past the tall tiles' 32-bit offsets (384 rows x 6,000,000 elements), and past
+    those of the resource over all rows of a batch: bitwise the contiguous call's result."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    x, g, u = rnd((300, 128), 31), rnd((128, 128), 32, 0.1), rnd((128, 128), 33, 0.1)
+    outs = [torch.zeros(300, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    for xs, out in zip((x, _wide(x, 6_000_000)), outs):
+        _abi.call("pi0hip_tile_gated_ffn", xs.data_ptr(), xs.stride(0), W.packed_weight_ptr(g, 32),
+                  W.packed_weight_ptr(u, 32), out.data_ptr(), 128, 300, 128, 128, W._stream())
+    assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
+    x, g, u = rnd((256, 1024), 34), rnd((1024, 64), 35, 0.02), rnd((1024, 64), 36, 0.02)
+    outs = [torch.zeros(256, 64, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    for xs, out in zip((x, _wide(x, 9_000_000)), outs):
+        W.decoder_norm_gated_ffn(xs, g, u, out, None)
+    assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("M", [1025, 2049, 4097, 6201])
 def test_residual_blocks(M):
     K, N = 3072, 2048      # not a K of the whole-K kernel, which sums in another order

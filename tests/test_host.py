@@ -67,6 +67,22 @@ def test_rejected_arguments_do_not_launch():
         _abi.check(-2, "x")
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the pointers are made up: launches must fail")
+def test_wide_row_pitches_are_not_refused():
+    """Rows so far apart that a tall tile's 32-bit offsets would not reach: a shorter tile takes
+    the call (the launch itself fails here, for want of a device)."""
+    lib = _abi.lib()
+    wide, wider = 5_000_000, 9_000_000
+    for rc in (lib.pi0hip_tile_gated_ffn(16, wider, 16, 16, 16, 128, 300, 128, 128, None),
+               lib.pi0hip_tile_linear_bias_gelu(16, wider, 16, 16, 16, 256, 300, 256, 128, 256, 128, None),
+               lib.pi0hip_tile_linear(16, wide, 16, 16, 16, 3456, 3072, 3456, 1152, None),
+               lib.pi0hip_tile_linear_residual(16, wide, 16, 16, 2048, 6528, 2048, 3072, 1, None, 0, None),
+               lib.pi0hip_tile_linear_residual(16, wide, 16, 16, 2048, 6528, 2048, 16384, 1, None, 0, None),
+               lib.pi0hip_tile_qkv_rope(16, wide, 16, 16, 16, 16, 16, 256, 6528, 2048, 8, 256, None),
+               lib.pi0hip_norm_gated_ffn(16, wider, 16, 16, 16, 4096, 256, 4096, 1024, None)):
+        assert rc > 0
+
+
 ENCODER_OPS = {"encoder_projector", "encoder_norm_qkv_rope", "encoder_out_proj_residual",
                "encoder_norm_gated_ffn", "encoder_ffn_down_residual", "encoder_attention",
                "vision_patch_embed", "vision_norm_qkv", "vision_out_proj_residual",
