@@ -78,6 +78,109 @@ def check_kblock_waits(asm: str) -> list[str]:
     return bad
 
 
+def _kernels(asm: str, pattern: str):
+    """(name, events) of the kernels matching `pattern`. Events, in text order: "C" a buffer load
+    into LDS, "L" any other load, "R" an LDS read, "B" a barrier, ("V", n) / ("K", n) a wait that
+    leaves n vector-memory / LDS operations outstanding, "E" the end of the text."""
+    for m in re.finditer(rf"^(_ZN3pi0\d+(?:{pattern})I?\w*):", asm, re.M):
+        events = []
+        for ln in asm[m.end():asm.index("s_endpgm", m.end())].split("\n"):
+            ln = ln.split(";")[0].strip()
+            if ln.startswith(("global_load", "buffer_load")):
+                events.append("C" if ln.endswith(" lds") else "L")
+            elif ln.startswith("ds_read"):
+                events.append("R")
+            elif ln.startswith("s_barrier"):
+                events.append("B")
+            elif ln.startswith("s_waitcnt"):
+                for op, kind in (("vmcnt", "V"), ("lgkmcnt", "K")):
+                    w = re.search(rf"\b{op}\((\d+)\)", ln)
+                    if w:
+                        events.append((kind, int(w.group(1))))
+        yield m.group(1), events + ["E"]
+
+
+# kernels whose waves read only what they copied themselves, in chunks of four copies that four
+# LDS reads consume, through four slots a wave
+_PRIVATE_CHUNKS = "rows32_res_kernel|qkv_rows32_kernel|gate_stream_kernel"
+
+
+def check_chunk_waits(asm: str) -> tuple[list[str], list[str]]:
+    """The kernels of _PRIVATE_CHUNKS (names with a wait that is too loose, names with a wait for
+    everything in flight before the last chunk).
+
+    Vector-memory operations complete in issue order, so at a wait vmcnt(N) all but the N newest
+    have landed: the last copy of a chunk must be among those when the chunk is read, and a copy
+    into a slot must follow the completed reads of the chunk that the slot held."""
+    loose, full = [], []
+    for name, events in _kernels(asm, _PRIVATE_CHUNKS):
+        issued = landed = reads = read_done = 0
+        copies, ok, drained = [], True, False
+        for e in events[:events.index("B")]:
+            if e in ("C", "L"):
+                if e == "C":
+                    ok &= len(copies) // 4 < 4 or read_done >= (len(copies) // 4 - 3) * 4
+                    copies.append(issued)
+                issued += 1
+            elif e == "R":
+                last = reads // 4 * 4 + 3
+                ok &= last < len(copies) and copies[last] < landed
+                reads += 1
+            elif e[0] == "V":
+                drained |= e[1] == 0 and reads // 4 + 1 < len(copies) // 4
+                landed = max(landed, issued - e[1])
+            elif e[0] == "K":
+                read_done = max(read_done, reads - e[1])
+        if not ok or reads != len(copies) or not copies:
+            loose.append(name)
+        if drained:
+            full.append(name)
+    return loose, full
+
+
+# kernels whose k loop shares its copies between waves, a wait and a barrier per step, and the
+# steps that may still be in flight at a wait of a loop unrolled over n steps
+_SHARED_STEPS = {"tile_gemm_kernel": lambda n: n - 2,    # step s read next, up to s + n - 2 issued
+                 "block_gemm_kernel": lambda n: n - 2,   # s + 1 read next, s + n - 1 issued
+                 "enc_attn_wide_kernel": lambda n: 1}    # b + 1 read next, b + 2 issued
+
+
+def check_step_waits(asm: str) -> list[str]:
+    """Names of the kernels of _SHARED_STEPS whose k loop waits for less than the copies of the
+    step behind the barrier and the reads of the slot that is filled next, or for more."""
+    bad = []
+    for kernel, in_flight in _SHARED_STEPS.items():
+        strip = kernel == "tile_gemm_kernel"             # weights to registers, not to LDS
+        for name, events in _kernels(asm, kernel):
+            waits = {}                                   # barrier -> its wait's vmcnt
+            for i, e in enumerate(events):
+                if e == "B":
+                    waits.update({i: v[1] for v in events[i - 2:i] if v[0] == "V"})
+            steps = sorted(waits)
+            end = events.index(("V", 0), steps[0])       # everything lands before the epilogue
+            steps = [i for i in steps if i < end]
+            loop = events[steps[0]:end]
+            lead = None if strip else steps.pop(0)       # the wait in front of the loop
+            n, copies, loads = len(steps), loop.count("C"), loop.count("L")
+            if n == 0 or copies == 0 or copies % n or loads % n:
+                bad.append(name)
+                continue
+            copies, loads = copies // n, loads // n
+            # a strip's weight loads of the step itself are waited for where they are used
+            bound = in_flight(n) * (copies + loads) + (loads if strip else 0)
+            ok = all(waits[i] == bound for i in steps)
+            for i, j in zip(steps, steps[1:]):
+                ok &= events[i:j].count("C") == copies and events[i:j].count("L") == loads
+            if strip:                                    # a step's copies before its weights
+                ok &= all("L" not in events[i:events.index("C", i)] for i in steps)
+            else:
+                ok &= all(events[i - 1] == ("K", 0) for i in steps)
+                ok &= waits[lead] <= events[:lead].count("C") - copies
+            if not ok:
+                bad.append(name)
+    return bad
+
+
 # kernels whose every copy lies inside its resource, whatever the call's sizes
 _COPIES_IN_RANGE = ("enc_attn_wide_kernel",)      # clamped blocks of the packed K and V^T
 
@@ -113,7 +216,7 @@ def scratch_kernels(asm: str) -> list[str]:
 def check_device_code(src: str) -> None:
     """Compile `src` to device assembly and fail if any packed fp32 VALU op was
     generated, if any kernel uses scratch memory, if a copy into LDS could leave its
-    resource's range check, or (pi0_gemm.hip) if a skinny GEMM's k-block waits are unsafe."""
+    resource's range check, or if a counted wait does not cover the copies it stands for."""
     cmd = [HIPCC, *FLAGS, "--cuda-device-only", "-S", src, "-o", "-"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
@@ -126,6 +229,9 @@ def check_device_code(src: str) -> None:
     loose = unchecked_copies(res.stdout)
     if loose:
         raise RuntimeError(f"{src}: LDS copies outside the range check in {loose}")
+    waits = check_chunk_waits(res.stdout)[0] + check_step_waits(res.stdout)
+    if waits:
+        raise RuntimeError(f"{src}: counted waits do not match the LDS copies in {waits}")
     if os.path.basename(src) == "pi0_gemm.hip":
         bad = check_kblock_waits(res.stdout)
         if bad:
