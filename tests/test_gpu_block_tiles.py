@@ -1,4 +1,4 @@
-"""The 8-wave block GEMMs at ragged row counts, one per tile that the dispatch can pick.
+"""The 8-wave block GEMMs and the batched decoder's kernels at ragged row counts.
 
 Every tile accumulates each output over k in the same order, so a call's rows must be, bit for
 bit, those of the same entry called on at most 200 of them at a time (which the strip tiles
@@ -84,9 +84,10 @@ def test_residual_blocks(M):
 
 
 @pytest.mark.parametrize("K", [2048, 4096])
-@pytest.mark.parametrize("M", [65, 96, 204, 257, 511])
+@pytest.mark.parametrize("M", [65, 96, 204, 225, 255, 256, 257, 511])
 def test_whole_k_residual(M, K):
-    """32 x 32 outputs over the whole K, against a 64-bit product: bf16 rounding of the output
+    """32 x 32 outputs over the whole K (up to 256 rows at N = 1024; past it the unsplit 32 x 128
+    strip), against a 64-bit product: bf16 rounding of the output
     alone is 2^-9 of a value, the fp32 sums' order adds 1e-6 of the row's scale."""
     if not torch.cuda.is_available():
         pytest.skip("needs a GPU")
@@ -196,7 +197,7 @@ def test_batched_gate_rows(M):
     assert torch.all(out[M:] == 7.0), "stored past row M"
 
 
-@pytest.mark.parametrize("B,L", [(3, 769), (8, 256), (5, 415), (2, 815)])
+@pytest.mark.parametrize("B,L", [(3, 769), (8, 256), (5, 415), (2, 1024), (2, 815)])
 @pytest.mark.parametrize("scale", [1.0, 6.0])           # ordinary, nearly one-hot
 def test_encoder_attention_many_rows(B, L, scale):
     """The 128-row workgroups (from 128 of them on; the last case stays below) against 64 bits:
@@ -215,3 +216,66 @@ def test_encoder_attention_many_rows(B, L, scale):
     # bf16 logits: 2^-9 of a logit of about 4 scale, so 4 scale 2^-9 on P
     assert err <= (4e-3 if wide else 4e-3 + scale * 2.0 ** -7), err
     assert torch.isfinite(out).all()
+
+
+def _same_specials(out, ref, tol):
+    """NaN where the reference has NaN, its infinities, and elsewhere its values within tol."""
+    out, ref = out.double(), ref.double()
+    assert torch.equal(out.isnan(), ref.isnan())
+    inf = ref.isinf()
+    assert torch.equal(out[inf], ref[inf])
+    ok = ~inf & ~ref.isnan()
+    assert ok.any() and torch.all((out[ok] - ref[ok]).abs() <= tol * ref[ok].abs().max())
+
+
+def _gelu(v):
+    return 0.5 * v * (1.0 + torch.tanh(0.7978845608028654 * (v + 0.044715 * v ** 3)))
+
+
+@pytest.mark.parametrize("entry,M,K,N", [
+    ("gated", 300, 128, 128),              # 192-row blocks
+    ("residual", 2100, 384, 2048),         # 128 x 256 blocks
+    ("residual", 96, 2048, 128),           # 32 x 32 outputs over the whole K
+    ("decoder gate", 130, 1024, 64)])      # rows streamed past a column tile
+def test_non_finite_rows(entry, M, K, N):
+    """A row with a NaN or an infinity gives what the formula gives, and no other row notices."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    x, w, u, r0 = rnd((M, K), 37), rnd((K, N), 38, 0.05), rnd((K, N), 39, 0.05), rnd((M, N), 40)
+    for row, v in ((1, float("nan")), (33, float("inf")), (65, -float("inf")), (M - 1, float("inf"))):
+        x[row, (7 * row) % K] = v
+    out = r0.clone()
+    xd = x.double()
+    if entry == "residual":
+        _abi.call("pi0hip_tile_linear_residual", x.data_ptr(), K, W.packed_weight_ptr(w, 32),
+                  out.data_ptr(), N, M, N, K, 1, None, 0, W._stream())
+        ref = xd @ w.double() + r0.double()
+    elif entry == "gated":
+        _abi.call("pi0hip_tile_gated_ffn", x.data_ptr(), K, W.packed_weight_ptr(w, 32),
+                  W.packed_weight_ptr(u, 32), out.data_ptr(), N, M, N, K, W._stream())
+        ref = _gelu(xd @ w.double()) * (xd @ u.double())
+    else:
+        W.decoder_norm_gated_ffn(x, w, u, out, None)
+        f = torch.rsqrt(xd.square().mean(1, keepdim=True) + 1e-6).bfloat16().double()
+        ref = _gelu(f * (xd @ w.double())) * (f * (xd @ u.double()))
+    _same_specials(out, ref, 2.0 ** -7)     # the bf16 result, and the row factor's rounding twice
+
+
+@pytest.mark.parametrize("B,L", [(2, 1024), (1, 100)])        # 128-row workgroups, 32-row ones
+def test_encoder_attention_non_finite(B, L):
+    """Keys with an infinity (weight 0 or NaN by the query's sign), a NaN query, an infinite V."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    from flash_vla_amd.arena import ScratchPool
+    from flash_vla_amd.backends.hip import encoder_wrappers as EW
+    q, k, v = rnd((B * L * 8, 256), 41), rnd((B, L, 256), 42), rnd((B, L, 256), 43)
+    q[:, 5] = q[:, 5].abs() + 0.1
+    q[3, 5] = -1.0                          # the one query that the key below attracts
+    q[9, 0] = float("nan")
+    k[:, 40, 5] = -float("inf")
+    v[:, 70, 200] = float("inf")
+    with W.use_pool(ScratchPool()):
+        out = EW.encoder_attention(q, k, v, 1 / 16).reshape(B, L * 8, 256)
+    p = torch.softmax(q.double().reshape(B, L * 8, 256) @ k.double().transpose(1, 2) / 16, -1)
+    # P's 2^-9 roundings average out, the narrow form's bf16 logits add 4 x 2^-9
+    _same_specials(out, p @ v.double(), 2.0 ** -5)

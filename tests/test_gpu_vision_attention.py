@@ -33,3 +33,24 @@ def test_against_64_bits(views, scale):
         out = VW.vision_attention(qkv)
     ref = _ref(qkv)
     assert torch.all((out.double() - ref).abs() <= 2.0 ** -7 * ref.abs().amax(-1, keepdim=True))
+
+
+def test_non_finite():
+    """A key with an infinity (weight 0 or NaN by the query's sign), a NaN query, an infinite V:
+    what the formula gives, in their own head and view alone."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    g = torch.Generator(device="cuda").manual_seed(7)
+    qkv = torch.randn(2, 256, 3456, generator=g, device="cuda")
+    qkv[0, :, 72 + 3] = qkv[0, :, 72 + 3].abs() + 0.1     # head 1's queries, dim 3
+    qkv[0, 200, 72 + 3] = -1.0
+    qkv[0, 150, 1152 + 72 + 3] = -float("inf")
+    qkv[0, 30, 5 * 72] = float("nan")
+    qkv[1, 250, 2304 + 15 * 72 + 71] = float("inf")
+    qkv = qkv.bfloat16()
+    with W.use_pool(ScratchPool()):
+        out = VW.vision_attention(qkv).double()
+    ref = _ref(qkv)
+    assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
+    ok = ref.isfinite()
+    assert torch.all((out[ok] - ref[ok]).abs() <= 2.0 ** -7 * ref[ok].abs().max())
