@@ -498,9 +498,10 @@ __global__ __launch_bounds__(256, 1) void qkv_rows32_kernel(GemmArgs a) {
 // and its x blocks pass through 16 KB of LDS in four 64-deep chunks, each refilled with the
 // next block's as soon as its fragments are read. Each output's arithmetic is
 // skinny_gemm_kernel's, so a request's rows are bitwise those of a batch of one. Each further
-// 64 rows cost a refill's round trip, 2 us, which is where the tiles take over. Cold weights,
-// us against the tiles: 66 rows 9.4 (13.1), 102 9.6 (13.2), 153 11.6 (13.4), 204 13.2 (13.4),
-// 306 19.2 (17.6).
+// 64 rows cost 2 us: the compiler does not tell the slot refilled last from the one read next
+// and waits for all four chunks before each block's first, so a block pays a whole round trip.
+// The tiles take over at 257 rows. Cold weights, us against the tiles: 66 rows 9.4 (13.1), 102
+// 9.6 (13.2), 153 11.6 (13.4), 204 13.2 (13.4), 306 19.2 (17.6).
 template <int NB>     // 32-row blocks per wave
 __global__ __launch_bounds__(512, 1) void gate_stream_kernel(GemmArgs a) {
   constexpr int KTW = 8, NKG = 4, NCH = 4;

@@ -20,8 +20,9 @@ from ...arena import ScratchPool
 from . import _abi
 
 DECODER_HEADS = 8
-# Above one 64-row block (the batched decoder, M = B x 51) the decoder's GEMMs run on the
-# prefix encoder's tile kernel: the skinny kernel would stream the weights once per row block.
+# Above one 64-row block (the batched decoder, M = B x 51) the decoder's residual GEMMs, and
+# its gated FFN past 256 rows, run on the prefix encoder's kernels: the skinny kernel would
+# stream the weights once per row block.
 _TILE_M = 64
 _POOL = ScratchPool()
 
@@ -454,7 +455,7 @@ def _residual(x, weight, out, role):
                   _ptr(out), out.stride(0), M, N, K, _stream())
         return out
     if M > _TILE_M and K % 256 == 0 and N % 128 == 0:
-        # the decoder's two K have a kernel that needs no split over workgroups
+        # the model's two K need no split over workgroups; other widths keep four splits
         s = 1 if K in (2048, 4096) else 4
         nbytes = _abi.lib().pi0hip_tile_workspace_bytes(M, N, s)
         ws = (scratch(f"tile_ws_{role}", (nbytes,), torch.uint8, x.device).data_ptr()
