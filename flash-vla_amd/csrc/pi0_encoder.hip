@@ -9,7 +9,8 @@
 //     fragment order. One barrier per 64-deep step.
 //   * tiles are assigned so that the workgroups dispatched to one XCD (the
 //     hardware deals workgroups round-robin over the 8 XCDs) cover consecutive
-//     tiles -- all row blocks of a weight column block -- so each weight block
+//     tiles -- all row blocks of a weight column block, or of a group of them
+//     where the rows are many (tile_group) -- so each weight block
 //     is read into one XCD's L2 once.
 //   * split-K (ffn-down, K = 16384) writes fp32 partials and a second launch
 //     sums them in split order and applies the residual epilogue.
@@ -1372,11 +1373,14 @@ using namespace pi0;
 // ---- host-side launch helpers ----------------------------------------------------
 
 // Column tiles per group of the tile order (tile_of): as many as balance the rows and columns
-// of the 32 tiles that an XCD holds. Up to 1024 rows the plain order is as good or better (816
-// rows, an encoder pass: 560.5 us plain, 562.4 grouped); past it grouping measured
-// 873 -> 859 us (two encoder layers, 3264 rows) and 570 -> 551 us (three vision layers, 3072).
+// of the 32 tiles that an XCD holds, from 1536 rows on. us per launch in the plain order /
+// grouped (cold weights): 3072 rows vision QKV 36.2 / 31.7, encoder down 209 / 189; 6528 rows
+// encoder gate 748 / 711, QKV 81.7 / 76.0; 4096 rows vision down 78.0 / 65.7; 1536 rows vision
+// QKV 18.4 / 17.9, encoder o-proj 19.2 / 18.4. Below that few row tiles share the columns and
+// the groups cost more than they save: 1280 rows vision QKV 18.2 / 20.0, FFN-up 21.4 / 22.3,
+// 1072 rows encoder gate 139 / 145, 1024 rows vision QKV 12.5 / 13.1; 816 rows are level.
 static int tile_group(const TileArgs& a, int bm, int bn) {
-  if (a.M <= 1024) return 1;
+  if (a.M < 1536) return 1;
   return std::max(1, std::min(a.tiles_n, (int)lroundf(sqrtf(32.f * bm / bn))));
 }
 
@@ -1506,7 +1510,7 @@ static int linear_launch(const TileArgs& a, hipStream_t s) {
 
 // Split-K partials of a residual GEMM (round lengths at 4096 of K per split).
 static int partial_launch(const TileArgs& a, hipStream_t s) {
-  // small M (the batched decoder, 204 rows): 32-row tiles, two workgroups per CU
+  // small M (the encoder down of one view without a prompt): 32-row tiles, two workgroups per CU
   if (a.M <= 256) return launch_tile_auto<32, 32, 4, TE_PARTIAL, false, 2>(a, s);
   switch (least({tile_us(a, 192, 128, 57.f),
                  block_us(a, 128, 256, 62.f),
@@ -1581,9 +1585,10 @@ int pi0hip_tile_linear_residual(const void* x, int ldx, const void* w_packed, vo
         return launch_block<4, 2, 2, 4, TE_RES>(a, s);
       return launch_tile_d4<128, 64, TE_RES, false>(a, s);
     }
-    // The batched decoder's o-proj and down (N = 1024, K 2048 / 4096): 32 x 32 workgroups over
-    // the whole K, 204 rows 8.5 -> 4.9 and 11.2 -> 8.1 against 4 splits and their sum, 408
-    // rows 15.5 -> 8.1 and 20.8 -> 14.8.
+    // The batched decoder's o-proj and down (N = 1024, K 2048 / 4096), against 4 splits and
+    // their sum: up to 256 rows, one round of them, 32 x 32 workgroups over the whole K, 204
+    // rows 8.5 -> 4.9 and 11.2 -> 8.1; past it 32 x 128 strips, 408 rows 15.5 -> 8.1 and
+    // 20.8 -> 14.8.
     const bool rows32 = (K == 2048 || K == 4096) && N % 128 == 0;   // whole tiles, as the others
     switch (least({tile_us(a, 64, 128, 13.3f), block_us(a, 128, 128, 20.5f),
                    block_us(a, 128, 256, 28.5f), block_us(a, 192, 256, 42.f),
