@@ -42,7 +42,7 @@ GATE_BYTES = 2 * 1024 * 4096 * 2           # gate + up weights of one layer (act
 # HBM bytes per launch from rocprofv3 FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 (KiB; factors from a
 # plain 256 MiB copy); profiles/kernels_hbm_traffic_config2_config3.md
 GATE_TRAFFIC_BYTES = (8645.0 * 2.0 + 408.0 * 1.0) * 1024
-ENC_GATE_TRAFFIC_BYTES = (77975.5 * 2.0 + 24576.0 * 1.0) * 1024
+ENC_GATE_TRAFFIC_BYTES = (77941.8 * 2.0 + 24576.0 * 1.0) * 1024   # block_gemm_kernel at M = 768
 
 
 def _time_graph(run, n_inner, reps, torch):
