@@ -1221,6 +1221,9 @@ struct VisAttnArgs {
 
 constexpr int VA_QT = 2, VA_KS = 2;                     // query tiles, key parts per workgroup
 
+// WIDE: rows too far apart for 32-bit offsets over a whole view; every copy then has a resource
+// of its own, from its first row on.
+template <bool WIDE>
 __global__ __launch_bounds__(64 * VA_QT * VA_KS, 1) void vision_attn_kernel(VisAttnArgs a) {
   constexpr int QT = VA_QT, KS = VA_KS, NW = QT * KS, CH = VA_HD / 8, WORDS = VA_TOK * CH, CI = WORDS / (64 * NW);
   constexpr int NB = VA_TOK / 32 / KS;                  // 32-key blocks of a wave
@@ -1232,18 +1235,31 @@ __global__ __launch_bounds__(64 * VA_QT * VA_KS, 1) void vision_attn_kernel(VisA
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6), qi = wave / KS, kp = wave % KS;
   const int head = blockIdx.y, view = blockIdx.z;
   const __bf16* base = a.qkv + (size_t)view * VA_TOK * a.ldqkv + head * VA_HD;
-  const int nbytes = ((VA_TOK - 1) * a.ldqkv + VA_HD) * (int)sizeof(__bf16);
-  const __amdgpu_buffer_rsrc_t kr = rows_rsrc_sgpr(base + a.dim, nbytes);
-  const __amdgpu_buffer_rsrc_t vr = rows_rsrc_sgpr(base + 2 * a.dim, nbytes);
-  int off[CI];
+  if constexpr (WIDE) {
 #pragma unroll
-  for (int i = 0; i < CI; ++i) {
-    const int id = (i * NW + wave) * 64 + lane, row = id / CH;
-    off[i] = (row * a.ldqkv + (id - row * CH) * 8) * (int)sizeof(__bf16);
-    buf_load16_lds(kr, &kv[(i * NW + wave) * 64], off[i]);
+    for (int i = 0; i < 2 * CI; ++i) {                  // K, then V
+      const int w0 = (i % CI * NW + wave) * 64, row0 = w0 / CH, row = (w0 + lane) / CH;
+      const __bf16* src = base + (i < CI ? 1 : 2) * a.dim + (size_t)row0 * a.ldqkv;
+      const int rows = min(63 / CH + 2, VA_TOK - row0); // that a copy's 64 chunks can touch
+      const __amdgpu_buffer_rsrc_t r =
+          rows_rsrc_sgpr(src, ((rows - 1) * a.ldqkv + VA_HD) * (int)sizeof(__bf16));
+      buf_load16_lds(r, &kv[(i < CI ? 0 : WORDS) + w0],
+                     ((row - row0) * a.ldqkv + (w0 + lane - row * CH) * 8) * (int)sizeof(__bf16));
+    }
+  } else {
+    const int nbytes = ((VA_TOK - 1) * a.ldqkv + VA_HD) * (int)sizeof(__bf16);
+    const __amdgpu_buffer_rsrc_t kr = rows_rsrc_sgpr(base + a.dim, nbytes);
+    const __amdgpu_buffer_rsrc_t vr = rows_rsrc_sgpr(base + 2 * a.dim, nbytes);
+    int off[CI];
+#pragma unroll
+    for (int i = 0; i < CI; ++i) {
+      const int id = (i * NW + wave) * 64 + lane, row = id / CH;
+      off[i] = (row * a.ldqkv + (id - row * CH) * 8) * (int)sizeof(__bf16);
+      buf_load16_lds(kr, &kv[(i * NW + wave) * 64], off[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < CI; ++i) buf_load16_lds(vr, &kv[WORDS + (i * NW + wave) * 64], off[i]);
   }
-#pragma unroll
-  for (int i = 0; i < CI; ++i) buf_load16_lds(vr, &kv[WORDS + (i * NW + wave) * 64], off[i]);
   __builtin_amdgcn_sched_barrier(0);
   // Q^T fragments: lane holds Q[q][16 kk + 8 h .. + 7] (zero past d = 72)
   const int q = (blockIdx.x * QT + qi) * 32 + r;
@@ -1812,16 +1828,18 @@ int pi0hip_vision_attention(const void* qkv, int ldqkv, void* out, int ldo, int 
   if (!qkv || !out || views <= 0 || heads <= 0) return PI0HIP_ERR_ARG;
   const int dim = heads * head_dim;
   if (tokens != VA_TOK || head_dim != VA_HD || ldqkv < 3 * dim || ldo < dim ||
-      misaligned(qkv, ldqkv) || (ldo & 3) || (reinterpret_cast<uintptr_t>(out) & 7) ||
-      (long long)VA_TOK * ldqkv * (long long)sizeof(__bf16) > INT_MAX)
+      misaligned(qkv, ldqkv) || (ldo & 3) || (reinterpret_cast<uintptr_t>(out) & 7))
     return PI0HIP_ERR_SHAPE;
   VisAttnArgs a = {};
   a.qkv = (const __bf16*)qkv; a.ldqkv = ldqkv;
   a.out = (__bf16*)out; a.ldo = ldo;
   a.dim = dim;
   a.scale_log2 = 1.4426950408889634f * scale;
-  hipLaunchKernelGGL(vision_attn_kernel, dim3(VA_TOK / (32 * VA_QT), heads, views),
-                     dim3(64 * VA_QT * VA_KS), 0, s, a);
+  const dim3 grid(VA_TOK / (32 * VA_QT), heads, views), block(64 * VA_QT * VA_KS);
+  if ((long long)VA_TOK * ldqkv * (long long)sizeof(__bf16) > INT_MAX)
+    hipLaunchKernelGGL(vision_attn_kernel<true>, grid, block, 0, s, a);
+  else
+    hipLaunchKernelGGL(vision_attn_kernel<false>, grid, block, 0, s, a);
   return (int)hipGetLastError();
 }
 

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from flash_vla_amd.arena import ScratchPool
+from flash_vla_amd.backends.hip import _abi
 from flash_vla_amd.backends.hip import vision_wrappers as VW
 from flash_vla_amd.backends.hip import wrappers as W
 
@@ -54,3 +55,20 @@ def test_non_finite():
     assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
     ok = ref.isfinite()
     assert torch.all((out[ok] - ref[ok]).abs() <= 2.0 ** -7 * ref[ok].abs().max())
+
+
+def test_wide_row_pitch():
+    """Rows 5,000,000 elements apart, past 32-bit offsets over a view: bitwise the packed result."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    g = torch.Generator(device="cuda").manual_seed(8)
+    qkv = torch.randn(256, 3456, generator=g, device="cuda").bfloat16()
+    pitch = 5_000_000
+    wide = torch.empty(256 * pitch, dtype=torch.bfloat16, device="cuda").view(256, pitch)[:, :3456]
+    wide.copy_(qkv)
+    outs = [torch.zeros(256, 1152, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    for t, out in zip((qkv, wide), outs):
+        _abi.call("pi0hip_vision_attention", t.data_ptr(), t.stride(0), out.data_ptr(), 1152, 1, 256,
+                  16, 72, 72 ** -0.5, None, 0, W._stream())
+    assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
+    torch.cuda.empty_cache()

@@ -79,6 +79,7 @@ def test_wide_row_pitches_are_not_refused():
                lib.pi0hip_tile_linear_residual(16, wide, 16, 16, 2048, 6528, 2048, 3072, 1, None, 0, None),
                lib.pi0hip_tile_linear_residual(16, wide, 16, 16, 2048, 6528, 2048, 16384, 1, None, 0, None),
                lib.pi0hip_tile_qkv_rope(16, wide, 16, 16, 16, 16, 16, 256, 6528, 2048, 8, 256, None),
+               lib.pi0hip_vision_attention(16, wide, 16, 1152, 1, 256, 16, 72, 0.1, None, 0, None),
                lib.pi0hip_norm_gated_ffn(16, wider, 16, 16, 16, 4096, 256, 4096, 1024, None)):
         assert rc > 0
 
